@@ -1,6 +1,5 @@
-// GEMM on fp32 / fp16 / bf16 and K-quant (Q4_K, Q5_K, Q6_K) weights on the fp32
-// matrix cores: out[r][c] = sum_i x[r][i] * w(c, i), the weights decoded exactly to
-// fp32 as they are staged.
+// GEMM on fp32 / fp16 / bf16 and K-quant (Q4_K, Q5_K, Q6_K) weights: out[r][c] = sum_i
+// x[r][i] * w(c, i), the weights decoded exactly.
 //
 // Reference: hip_matmul (matmul_kernel<float>, src/hip_ops.hip:43-64), hip_matmul_u16
 // (matmul_kernel<uint16_t>: fp16/bf16 weights widened exactly) and hip_matmul_qk
@@ -10,9 +9,10 @@
 // fp32 sums in k order; weights w(c, i) = element c*k + i of the flat weight array
 // (row-major [n][k]; K-quant superblocks cover 256 consecutive elements).
 //
-// Design for gfx950: the fp32 matrix-core tile kernel of gemm_tile.hpp for m > 16
-// (m <= 32 takes 32-row tiles, so a small m does not multiply the matrix-core work),
-// and the weight-streaming decode products below for m <= 16.  The sums are fp32
+// Design for gfx950: activations and weights of one 16-bit type go to the 16-bit matrix
+// cores as they are (gemm16.hpp, m > 2); otherwise the tile kernels of gemm_tile.hpp
+// for m > 16 (m <= 32 takes 32-row tiles, so a small m does not multiply the
+// matrix-core work), and the weight-streaming decode products below for m <= 16.  The sums are fp32
 // in a different order from the reference's, so results agree within the
 // recursive-summation bound the tests state.
 
@@ -21,6 +21,15 @@
 #include "gemm_tile.hpp"
 
 namespace nvf {
+
+// gemm16.hip: x and W of one 16-bit type, 16-byte aligned, k a multiple of 8
+int gemm16(const void* x, const void* w, bool bf16, void* out, int out_dtype, int64_t m, int64_t n, int64_t k,
+           hipStream_t st);
+
+template <typename TO>
+constexpr int dtype_of() {
+  return sizeof(TO) == 4 ? NVF_F32 : __is_same(TO, __bf16) ? NVF_BF16 : NVF_F16;
+}
 
 // ---------------------------------------------------------------------------
 // 32-element group sources for the decode products: one lane decodes a whole
@@ -200,6 +209,7 @@ struct GemvPrefetch<Q6KGroup> {
 // 2 < m <= 16: gemv_mfma_kernel (gemm_tile.hpp, v_mfma_f32_16x16x4_f32) with the
 // plain problem policy.
 constexpr int kGemvRows = 16;
+constexpr int kGemvFmaRows = 2;
 
 // Column sets / groups per wave: 4 (dense) or 2 (K-quants, larger runs) when that
 // leaves >= ~1000 workgroups, fewer for narrow outputs.
@@ -267,12 +277,29 @@ struct GemvSource<Q6K<8>> {
   static type make(const Q6K<8>& s) { return type{s.wq}; }
 };
 
+// Activations and dense weights of one 16-bit type: the 16-bit matrix-core GEMM.
+template <typename TX, typename Src>
+struct SameType16 {
+  static constexpr bool value = false;
+};
+template <typename T>
+struct SameType16<T, Table<8, T>> {
+  static constexpr bool value = sizeof(T) == 2;
+};
+
 template <typename TX, typename Src, typename TO>
 int launch_dense(const void* x, const Src& src, void* out, int64_t m, int64_t n, int64_t k, bool vec,
                  hipStream_t st) {
   const int tiles_n = (int)((n + kDgBN - 1) / kDgBN);
   const TX* xp = static_cast<const TX*>(x);
   TO* op = static_cast<TO*>(out);
+  if constexpr (SameType16<TX, Src>::value) {
+    // 16-byte chunks of k, and row offsets inside a tile within 31 bits.  One or two rows
+    // stay on the plain-FMA product (bf16 37888 x 3584, us: m = 1 42.6, m = 2 54; this GEMM
+    // 49 from m = 3 on; 3584 x 18944: 26 and 32 against 37).
+    if (vec && m > kGemvFmaRows && k % 8 == 0 && k < (1 << 22))
+      return gemm16(x, src.table, __is_same(TX, __bf16), out, dtype_of<TO>(), m, n, k, st);
+  }
   // decode product: whole runs per row (8 elements for dense rows, a 32-element group for K-quants)
   if (vec && m <= kGemvRows && k % RunOf<typename GemvSource<Src>::type>::value == 0)
     return launch_gemv<TX>(xp, GemvSource<Src>::make(src), op, m, n, k, st);
@@ -287,7 +314,7 @@ int launch_dense(const void* x, const Src& src, void* out, int64_t m, int64_t n,
   } else {
     const dim3 g((unsigned)(((m + 127) / 128) * tiles_n));
     const PlainProb<128, TO> prob{op, m, n, k};
-    if constexpr (SplitTile<Src>::value) {  // fp16 / bf16 weights: the split product on the bf16 matrix cores
+    if constexpr (SplitTile<Src>::value && !SameType16<TX, Src>::value) {  // fp16 / bf16 weights: the split product on the bf16 matrix cores
       if (!ragged) {
         gemm_tile_split_kernel<TX><<<g, kDgThreads, 0, st>>>(xp, src, prob, k, tiles_n);
         return launch_status("dense_gemm (split)");
