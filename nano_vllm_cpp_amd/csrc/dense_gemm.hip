@@ -26,6 +26,10 @@ namespace nvf {
 int gemm16(const void* x, const void* w, bool bf16, void* out, int out_dtype, int64_t m, int64_t n, int64_t k,
            hipStream_t st);
 
+// kq_gemm.hip: K-quant W and 16-bit x, 16-byte aligned, k a multiple of 256
+int kq_gemm(const void* x, bool bf16, const void* w, int kind, int layout, void* out, int out_dtype, int64_t m,
+            int64_t n, int64_t k, hipStream_t st);
+
 template <typename TO>
 constexpr int dtype_of() {
   return sizeof(TO) == 4 ? NVF_F32 : __is_same(TO, __bf16) ? NVF_BF16 : NVF_F16;
@@ -332,6 +336,10 @@ template <typename TX, typename TO>
 int dispatch_weights(const void* x, const void* w, int w_format, int layout, void* out, int64_t m, int64_t n,
                      int64_t k, bool vec, hipStream_t st) {
   const uint8_t* wb = static_cast<const uint8_t*>(w);
+  if constexpr (sizeof(TX) == 2) {  // whole superblocks per row: the 16-bit matrix cores
+    if (w_format >= NVF_W_Q4_K && vec && m > kGemvRows && k % 256 == 0 && k < (1 << 22))
+      return kq_gemm(x, __is_same(TX, __bf16), w, w_format, layout, out, dtype_of<TO>(), m, n, k, st);
+  }
   switch (w_format) {
     case NVF_W_F32:
       return launch_dense<TX, Table<8, float>, TO>(x, Table<8, float>{static_cast<const float*>(w)}, out, m, n, k, vec, st);

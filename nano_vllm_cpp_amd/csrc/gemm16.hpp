@@ -36,6 +36,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t g16_rsrc(const void* base, int
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
 
+// One 1 KB transfer HBM -> LDS: lane l's 16 bytes at r[off + soff] go to dst + 16 l.  (A
+// function of its own: kernels that call the builtin from a template can lose their
+// launch stubs in the host pass.)
+__device__ __forceinline__ void g16_dma(__amdgpu_buffer_rsrc_t r, uint8_t* dst, uint32_t off, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, off, soff, 0, 0);
+}
+
 // Waits until at most N of this wave's vector-memory operations are outstanding
 // (lgkmcnt and expcnt untouched).
 template <int N>
@@ -125,9 +132,7 @@ __global__ __launch_bounds__(WM* WN* KG * 64) __attribute__((amdgpu_waves_per_eu
       const int t = wave * kDma + i;  // uniform
       uint32_t o = off[i];
       if (tail) o = (int64_t)st * BK + kchunk[i] < k ? o : 0x80000000u;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(t * kRpi < BM ? ra : rb,
-                                               (__attribute__((address_space(3))) void*)(ring + buf * kStage + t * 1024),
-                                               16, o, kb, 0, 0);
+      g16_dma(t * kRpi < BM ? ra : rb, ring + buf * kStage + t * 1024, o, kb);
     }
   };
 

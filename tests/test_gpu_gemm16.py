@@ -1,5 +1,6 @@
-"""GPU parity of the 16-bit matrix-core GEMM (activations and weights both fp16 or both
-bf16): every tile shape of its choice, at sizes with ragged rows, columns and K.
+"""GPU parity of the products on the 16-bit matrix cores: activations and weights both fp16
+or both bf16, and K-quant weights with 16-bit activations.  Every tile shape of the
+choices, at sizes with ragged rows, columns and K.
 
 Small integers make every fp32 partial sum exact, so any summation order gives the exact
 product: the outputs are compared bit for bit with the float64 product rounded once to
@@ -7,10 +8,12 @@ the output type.  The non-finite case checks that infinities and NaN land where 
 products and sums of the same operands put them."""
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
 from nano_vllm_cpp_amd import ops
+from tests import harness as H
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +78,68 @@ def test_non_finite_operands(gpu, dtype):
     out = ops.matmul(x, w, n, W[dtype], out_dtype=torch.float32).double()
     assert torch.equal(torch.isnan(out), torch.isnan(want))
     assert torch.equal(out[~torch.isnan(want)], want[~torch.isnan(want)])
+
+
+# ---------------------------------------------------------------------------
+# K-quant weights with 16-bit activations (kq_gemm.hip), whole superblocks per row
+# ---------------------------------------------------------------------------
+KQ = [(12, H.GGML), (12, H.HIP_LEGACY), (13, H.GGML), (14, H.GGML)]
+KQ_IDS = ["q4k", "q4k_legacy", "q5k", "q6k"]
+# the workgroup's rows beside each
+KQ_SIZES = [
+    (17, 130, 256),      # 32: one superblock, two columns in the last tile
+    (33, 129, 2304),     # 64
+    (65, 24577, 256),    # 128
+    (129, 24580, 512),   # 256, one row in the last tile
+]
+
+
+def kq_case(seed, m, n, k, dt, kind):
+    r = H.rng(seed)
+    return H.gen_act(r, (m, k), dt), H.gen_weights(r, n, k, kind)
+
+
+def kq_oracle(x, dt, w, kind, layout, m, n, k):
+    want, err = np.empty((m, n), np.float64), np.empty((m, n), np.float64)
+    H.oracle().orc_matmul_w(H.ptr(x), dt, H.ptr(w), kind, layout, m, n, k, H.ptr(want), H.ptr(err))
+    return want, err
+
+
+@pytest.mark.parametrize("kind,layout", KQ, ids=KQ_IDS)
+@pytest.mark.parametrize("dt", [H.F16, H.BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("m,n,k", KQ_SIZES)
+def test_kquant_within_fp32_sum_bound(gpu, kind, layout, dt, m, n, k):
+    print(f"[case] kq {kind}/{layout} {m}x{n}x{k} dt={dt}", flush=True)
+    x, w = kq_case(100 * kind + m, m, n, k, dt, kind)
+    want, err = kq_oracle(x, dt, w, kind, layout, m, n, k)
+    for out_dtype in (torch.float32, H.torch_dtype(dt)):
+        guard = torch.full((m * n + 64,), 7.0, dtype=out_dtype, device=gpu)
+        out = ops.matmul(H.to_dev(x, gpu, dt), H.to_dev(w, gpu), n, kind, qk_layout=layout, out_dtype=out_dtype,
+                         out=guard[32:32 + m * n].view(m, n))
+        got = out.double().cpu().numpy()
+        # the bound of fp32 sums of the decoded products, plus half an ulp of a 16-bit output
+        tol = err + (0.0 if out_dtype == torch.float32 else 0.5 * H.ulp(want, dt))
+        assert (np.abs(got - want) <= tol).all(), float((np.abs(got - want) / tol).max())
+        assert bool((guard[:32] == 7).all()) and bool((guard[32 + m * n:] == 7).all()), "wrote outside the output"
+
+
+@pytest.mark.parametrize("kind,layout", KQ, ids=KQ_IDS)
+@pytest.mark.parametrize("dt", [H.F16, H.BF16], ids=["f16", "bf16"])
+def test_kquant_non_finite_operands(gpu, kind, layout, dt):
+    m, n, k = 40, 150, 512
+    x, w = kq_case(7 * kind, m, n, k, dt, kind)
+    xt = H.to_dev(x, gpu, dt)
+    xt[3, 7], xt[9, 300], xt[20, 0] = float("inf"), float("-inf"), float("nan")
+    if dt == H.BF16:
+        xt[30, 5] = 3.0e38  # finite, but not times a sub-block's whole-number scale
+    blk = w.reshape(n * k // 256, -1)
+    d_at = 208 if kind == 14 else 0
+    blk[4 * 2 + 1, d_at:d_at + 2] = np.array([np.inf], np.float16).view(np.uint8)  # column 4's second superblock
+    want, _ = kq_oracle(H.to_host(xt), dt, w, kind, layout, m, n, k)
+    got = ops.matmul(xt, H.to_dev(w, gpu), n, kind, qk_layout=layout, out_dtype=torch.float32).double().cpu().numpy()
+    with np.errstate(over="ignore"):
+        want32 = want.astype(np.float32).astype(np.float64)
+    assert (np.isnan(got) == np.isnan(want32)).all()
+    assert (np.isposinf(got) == np.isposinf(want32)).all() and (np.isneginf(got) == np.isneginf(want32)).all()
+    fin = np.isfinite(want32)
+    assert np.allclose(got[fin], want32[fin], rtol=1e-4, atol=1e-3 * np.abs(want32[fin & (np.abs(want32) < 1e6)]).max())
