@@ -414,13 +414,13 @@ int nvf_paged_attention_ws(const void* q, void* out, const void* k_cache, const 
  * host: cu_seqlens_host [num_seqs + 1] (0, then each sequence's end; the last entry is
  * tokens), the packing that query_seq describes on the device (the reference's
  * cu_seqlens_q, include/nanovllm/context.hpp:8-25, built on the host by
- * ModelRunner::prepare_prefill, src/model_runner.cpp:43-128).  When every sequence
- * starts at a multiple of 128 tokens, every 128-token tile holds one sequence and the
- * launch for tokens of mixed tiles is not made.  Results equal nvf_paged_attention_ws's.
+ * ModelRunner::prepare_prefill, src/model_runner.cpp:43-128).  When no 128-token tile
+ * holds more than 8 sequences, the launch for the tokens of such tiles is not made.
+ * Results equal nvf_paged_attention_ws's.
  * Contract: cu_seqlens_host must describe exactly the packing of query_seq (token t
  * belongs to sequence s iff cu_seqlens_host[s] <= t < cu_seqlens_host[s + 1]).  Only
- * its monotonicity and end points are checked; if it claims 128-aligned sequences
- * that query_seq does not have, the tokens of the mixed tiles are left unwritten. */
+ * its monotonicity and end points are checked; if it hides tiles of more than 8
+ * sequences that query_seq has, the tokens of those tiles are left unwritten. */
 int nvf_paged_attention_seqs_ws(const void* q, void* out, const void* k_cache, const void* v_cache,
                                 const int32_t* query_seq, const int32_t* query_key_len, const int32_t* block_tables,
                                 const int32_t* cu_seqlens_host, int num_seqs, int64_t tokens, int q_heads,

@@ -86,8 +86,7 @@ __global__ __launch_bounds__(256) void store_kv_generic_kernel(const T* __restri
 //                    holds for keys 16u + 4h + {0..3, 8..11} are its B operand
 //                    for key step u once both operands index keys that way)
 // P is rounded to the cache dtype for the MFMA; the row sums use the fp32 P.
-// Tiles whose tokens span sequences (or are partial at a sequence switch) are
-// left to attn_wave_kernel, which applies the same predicate.
+// A tile whose tokens span sequences is walked run by run (fa_tile_runs below).
 constexpr int kFaHd = 128;
 constexpr int kFaBq = 128;                       // query tokens per workgroup
 constexpr int kFaBk = 64;                        // keys per chunk
@@ -121,23 +120,46 @@ struct Mfma16<_Float16> {
   }
 };
 
-// True iff every token of the kFaBq-token tile `tile` (those < tokens) belongs to
-// one sequence.  Evaluated per wave; every wave of a workgroup gets the same answer.
-__device__ __forceinline__ bool fa_tile_uniform(const int32_t* __restrict__ qseq, int64_t tokens, int64_t tile) {
-  const int lane = threadIdx.x & 63;
-  const int64_t t0 = tile * kFaBq;
-  const int32_t s0 = qseq[t0];
-  bool same = true;
-#pragma unroll
-  for (int i = 0; i < kFaBq / 64; ++i) {
-    const int64_t t = t0 + lane + 64 * i;
-    if (t < tokens) same = same && qseq[t] == s0;
+// A tile's runs are its maximal stretches of consecutive tokens of one sequence.  A tile
+// of at most kFaMaxRuns runs is taken by the tile kernels, run after run: in a packed
+// prefill a tile that spans sequences holds one's tail and the next one's first keys, so
+// its further runs are short.  (Token by token on the decode kernels, whose chain over a
+// long context is serial, prompts of 4096, 3001, 2048 and 777 tokens took 132 us of 366 for
+// the 384 tokens of three tiles: 366 -> 263 us at fp16, fp32 prompts of 3072, 1531 and 700
+// 1070 -> 810; 32 prompts of 64 tokens 61 -> 17.)  A run costs about 3.5 us of latency, so a
+// crowded tile is better spread over the decode kernel's workgroups: 100 prompts of 20
+// tokens (7 runs) 60 -> 33 us, 300 of 8 (16 runs) 76 -> 68 but 400 of 5, whose last tile has
+// 16, 63 -> 114.  Every wave of a workgroup gets the same answer.
+constexpr int kFaMaxRuns = 8;
+struct FaRuns {  // bit i: the tile's token i starts a run (token 0's bit is clear)
+  uint64_t lo, hi;
+  __device__ __forceinline__ bool taken() const { return __popcll(lo) + __popcll(hi) < kFaMaxRuns; }
+  // the first run start after token r, or the tile's end
+  __device__ __forceinline__ int end_after(int r, int end) const {
+    const uint64_t a = r < 63 ? lo >> (r + 1) << (r + 1) : 0;
+    const uint64_t b = r < 64 ? hi : r < 127 ? hi >> (r - 63) << (r - 63) : 0;
+    return a ? __builtin_ctzll(a) : b ? 64 + __builtin_ctzll(b) : end;
   }
-  return __all(same);
+};
+__device__ __forceinline__ FaRuns fa_tile_runs(const int32_t* __restrict__ qseq, int64_t tokens, int64_t tile) {
+  static_assert(kFaBq == 128, "two tokens per lane");
+  const int lane = threadIdx.x & 63;
+  const int64_t t = tile * kFaBq + lane, last = tokens - 1;  // past the end: the last token again, no start
+  const int32_t a = qseq[t < last ? t : last], b = qseq[t + 64 < last ? t + 64 : last];
+  const int32_t pa = __shfl_up(a, 1), pb = __shfl_up(b, 1);
+  const int32_t a63 = __builtin_amdgcn_readlane(a, 63);
+  return {__ballot(lane > 0 && a != pa), __ballot(b != (lane > 0 ? pb : a63))};
+}
+
+// This lane, from the hardware's count, opaque to the optimizer.
+__device__ __forceinline__ int fa_lane() {
+  int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  asm volatile("" : "+v"(lane));
+  return lane;
 }
 
 template <typename T, bool SPLIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void fa_prefill_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 : 3))) void fa_prefill_kernel(
     const T* __restrict__ q, T* __restrict__ out, const T* __restrict__ kc, const T* __restrict__ vc,
     const int32_t* __restrict__ qseq, const int32_t* __restrict__ qlen, const int32_t* __restrict__ tables,
     int64_t tokens, int q_heads, int kv_heads, int bs, int max_blocks, float scale_log2, int64_t q_stride,
@@ -145,32 +167,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
   using M = Mfma16<T>;
   using v8 = typename M::v8;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int half = lane >> 5;
   const int64_t bid = blockIdx.x;
   const int64_t tile = tiles - 1 - bid / q_heads;  // the longest tiles (latest positions) first
   const int h = (int)(bid % q_heads);
   const int64_t t0 = tile * kFaBq;
-  if (!fa_tile_uniform(qseq, tokens, tile)) return;  // the whole workgroup: left to attn_wave_kernel
-  const int64_t seq = qseq[t0];
+  const FaRuns runs = fa_tile_runs(qseq, tokens, tile);
+  if (!runs.taken()) return;  // the whole workgroup: left to the decode kernel
   const int kvh = h / (q_heads / kv_heads);
   const int64_t kv_stride = (int64_t)kv_heads * kFaHd;
-  const int32_t* tab = tables + seq * max_blocks;
+  const int tend = tokens - t0 < kFaBq ? (int)(tokens - t0) : kFaBq;
 
-  // the tile's longest key range (every wave computes the same value)
+  int r0 = 0;
+#pragma unroll 1
+  while (true) {  // the tile's runs [r0, r1)
+  // The lane is opaque here and again after the chunks, so that what follows from it is
+  // worked out anew rather than kept in registers (168 VGPRs: three workgroups per CU).
+  int lane = fa_lane();
+  const int half = lane >> 5;
+  // this lane's query (a column of S^T and O^T)
+  const int ql = 32 * wave + (lane & 31);
+  const int64_t tq = t0 + ql;
+  const int r1 = runs.end_after(r0, tend);
+  const int32_t* tab = tables + (int64_t)qseq[t0 + r0] * max_blocks;
+
+  // the run's longest key range (every wave computes the same value)
   float lmax = 0.0f;
 #pragma unroll
   for (int i = 0; i < kFaBq / 64; ++i) {
-    const int64_t t = t0 + lane + 64 * i;
-    if (t < tokens) lmax = fmaxf(lmax, (float)qlen[t]);
+    const int t = lane + 64 * i;
+    if (t >= r0 && t < r1) lmax = fmaxf(lmax, (float)qlen[t0 + t]);
   }
   const int Lmax = (int)wave_max(lmax);
   const int nchunks = (Lmax + kFaBk - 1) / kFaBk;
 
-  // this lane's query (a column of S^T and O^T)
-  const int64_t tq = t0 + 32 * wave + (lane & 31);
-  const bool q_ok = tq < tokens;
+  const bool q_ok = ql >= r0 && ql < r1;
   const int L = q_ok ? qlen[tq] : 0;
   // the smallest key count among the wave's queries (chunks below it need no mask)
   // (a wave with no query in range takes the masked path; its outputs are not stored)
@@ -247,7 +278,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
   for (int d = 0; d < kFaHd / 32; ++d) o[d] = f32x16{};
   float m = -INFINITY, l = 0.0f;
 
-  // this workgroup's chunks: all of the tile's, or split blockIdx.z's split_keys keys
+  // this workgroup's chunks: all of the run's, or split blockIdx.z's split_keys keys
   int c0 = 0, c1 = nchunks;
   if constexpr (SPLIT) {
     c0 = (int)blockIdx.z * (split_keys / kFaBk);
@@ -375,26 +406,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
     }
   }
 
+  const int lane_e = fa_lane(), half_e = lane_e >> 5, ql_e = 32 * wave + (lane_e & 31);
+  const bool ok_e = ql_e >= r0 && ql_e < r1;
+  const int64_t tq_e = t0 + ql_e;
   // O^T layout: lane column = query, dims 32 d + 8 (j/4) + 4 half + j%4
   if constexpr (SPLIT) {  // unnormalised partial O, running max (exp2 units) and sum
-    if (q_ok) {
-      const int64_t pi = (tq * q_heads + h) * gridDim.z + blockIdx.z;
+    if (ok_e) {
+      const int64_t pi = (tq_e * q_heads + h) * gridDim.z + blockIdx.z;
       float* po = part + pi * kFaHd;
 #pragma unroll
       for (int d = 0; d < kFaHd / 32; ++d)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-          st16(po + 32 * d + 8 * g + 4 * half,
+          st16(po + 32 * d + 8 * g + 4 * half_e,
                __builtin_bit_cast(u32x4, f32x4{o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]}));
-      if (half == 0) {
+      if (half_e == 0) {
         float* pml = part + tokens * q_heads * gridDim.z * kFaHd + 2 * pi;
         pml[0] = m;
         pml[1] = l;
       }
     }
-  } else if (q_ok) {
+  } else if (ok_e) {
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    T* orow = out + (tq * q_heads + h) * kFaHd;
+    T* orow = out + (tq_e * q_heads + h) * kFaHd;
 #pragma unroll
     for (int d = 0; d < kFaHd / 32; ++d)
 #pragma unroll
@@ -403,10 +437,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
         t4 v;
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = (T)(o[d][4 * g + e] * inv);
-        *reinterpret_cast<t4*>(orow + 32 * d + 8 * g + 4 * half) = v;
+        *reinterpret_cast<t4*>(orow + 32 * d + 8 * g + 4 * half_e) = v;
       }
   }
+  r0 = r1;
+  if (r0 >= tend) break;
+  __syncthreads();  // the next run's chunks reuse the LDS
+  }
 }
+
 
 // ---------------------------------------------------------------------------
 // fp32 caches (the reference's own KV dtype) on the fp32 matrix cores,
@@ -442,23 +481,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   const int64_t tile = tiles - 1 - bid / q_heads;  // the longest tiles (latest positions) first
   const int h = (int)(bid % q_heads);
   const int64_t t0 = tile * kFaBq;
-  if (!fa_tile_uniform(qseq, tokens, tile)) return;  // the whole workgroup: left to attn_wave_kernel
-  const int64_t seq = qseq[t0];
+  const FaRuns runs = fa_tile_runs(qseq, tokens, tile);
+  if (!runs.taken()) return;  // the whole workgroup: left to the decode kernel
   const int kvh = h / (q_heads / kv_heads);
   const int64_t kv_stride = (int64_t)kv_heads * kFaHd;
-  const int32_t* tab = tables + seq * max_blocks;
+  const int tend = tokens - t0 < kFaBq ? (int)(tokens - t0) : kFaBq;
+  // this lane's query (a column of S^T and O^T)
+  const int ql = 32 * wave + (lane & 31);
+  const int64_t tq = t0 + ql;
+
+  int r0 = 0;
+#pragma unroll 1
+  while (true) {  // the tile's runs [r0, r1)
+  const int r1 = runs.end_after(r0, tend);
+  const int32_t* tab = tables + (int64_t)qseq[t0 + r0] * max_blocks;
 
   float lmax = 0.0f;
 #pragma unroll
   for (int i = 0; i < kFaBq / 64; ++i) {
-    const int64_t t = t0 + lane + 64 * i;
-    if (t < tokens) lmax = fmaxf(lmax, (float)qlen[t]);
+    const int t = lane + 64 * i;
+    if (t >= r0 && t < r1) lmax = fmaxf(lmax, (float)qlen[t0 + t]);
   }
   const int Lmax = (int)wave_max(lmax);
   const int nchunks = (Lmax + kF32Bk - 1) / kF32Bk;
 
-  const int64_t tq = t0 + 32 * wave + (lane & 31);
-  const bool q_ok = tq < tokens;
+  const bool q_ok = ql >= r0 && ql < r1;
   const int L = q_ok ? qlen[tq] : 0;
   const float lmin = -wave_max(q_ok ? -(float)L : -INFINITY);
   const int Lmin = lmin < 2.0e9f ? (int)lmin : 0;
@@ -502,7 +549,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   for (int d = 0; d < 4; ++d) o[d] = f32x16{};
   float m = -INFINITY, l = 0.0f;
 
-  // this workgroup's chunks: all of the tile's, or split blockIdx.z's split_keys keys
+  // this workgroup's chunks: all of the run's, or split blockIdx.z's split_keys keys
   int c0 = 0, c1 = nchunks;
   if constexpr (SPLIT) {
     c0 = (int)blockIdx.z * (split_keys / kF32Bk);
@@ -604,7 +651,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
       st16(orow + 4 * r, __builtin_bit_cast(u32x4, f32x4{o[0][j] * inv, o[1][j] * inv, o[2][j] * inv, o[3][j] * inv}));
     }
   }
+  r0 = r1;
+  if (r0 >= tend) break;
+  __syncthreads();  // the next run's chunks reuse the LDS
+  }
 }
+
 
 // ---------------------------------------------------------------------------
 // The decode kernels' end: a workgroup is one (token, kv head) whose 4 waves each
@@ -776,7 +828,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   }
   if (t < 0 || t >= tokens) return;  // an order entry outside the batch: nothing to compute (uniform)
   // workgroup-uniform: the whole workgroup leaves (fa_prefill_kernel's tile)
-  if (SKIP && fa_tile_uniform(qseq, tokens, t / kFaBq)) return;
+  if (SKIP && fa_tile_runs(qseq, tokens, t / kFaBq).taken()) return;
   // The tiles' second launch (SKIP) has one workgroup per token, so that its many
   // exiting workgroups stay few, and walks the kv heads; otherwise the workgroup's
   // kv head (one trip).
@@ -979,7 +1031,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   const int64_t t = tok_major ? (int64_t)order[ti] : ti;
   if (t < 0 || t >= tokens) return;
   // workgroup-uniform: the whole workgroup leaves (fa_prefill_f32_kernel's tile)
-  if (SKIP && fa_tile_uniform(qseq, tokens, t / kFaBq)) return;
+  if (SKIP && fa_tile_runs(qseq, tokens, t / kFaBq).taken()) return;
   // as fa_decode_kernel: the tiles' second launch walks the kv heads per token
   const int kvh0 = SKIP ? 0 : tok_major ? (int)(blockIdx.x % kv_heads) : (int)(blockIdx.x / tokens);
   const int kvh1 = SKIP ? kv_heads : kvh0 + 1;
@@ -1118,7 +1170,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_wave_kernel(
     const T* __restrict__ q, T* __restrict__ out, const T* __restrict__ kc, const T* __restrict__ vc,
     const int32_t* __restrict__ qseq, const int32_t* __restrict__ qlen, const int32_t* __restrict__ tables,
     int64_t tokens, int q_heads, int kv_heads, int hd, int bs, int max_blocks, float scale, int64_t q_stride,
-    bool skip_uniform_tiles) {
+    bool skip_taken_tiles) {
   constexpr int N = Pack<T>::N;
   __shared__ float q_sh[kAttnWaves][64 * DPL];
   __shared__ float p_sh[kAttnWaves][64];
@@ -1128,7 +1180,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_wave_kernel(
   if (gw >= tokens * q_heads) return;  // whole waves only; no workgroup barrier below
   const int64_t t = gw / q_heads;
   const int h = (int)(gw - t * q_heads);
-  if (skip_uniform_tiles && fa_tile_uniform(qseq, tokens, t / kFaBq)) return;  // fa_prefill_kernel's
+  if (skip_taken_tiles && fa_tile_runs(qseq, tokens, t / kFaBq).taken()) return;  // fa_prefill_kernel's
   const int kvh = h / (q_heads / kv_heads);
   const int L = qlen[t];
   T* o = out + (t * q_heads + h) * hd;
@@ -1326,10 +1378,10 @@ template <typename T>
 int attention_dispatch(const void* q, void* out, const void* kc, const void* vc, const int32_t* qseq,
                        const int32_t* qlen, const int32_t* tables, int64_t tokens, int q_heads, int kv_heads, int hd,
                        int bs, int max_blocks, float scale, int64_t q_stride, int64_t max_query_len, void* ws,
-                       int64_t ws_bytes, hipStream_t st, bool aligned = false, const int32_t* order = nullptr) {
-  // aligned: every sequence starts at a multiple of kFaBq tokens (checked on the host
-  // from the caller's cu_seqlens), so every tile is uniform and the tiles' second
-  // launch, whose workgroups would all exit, is not made
+                       int64_t ws_bytes, hipStream_t st, bool taken = false, const int32_t* order = nullptr) {
+  // taken: no tile has more than kFaMaxRuns runs (counted on the host from the caller's
+  // cu_seqlens), so the tile kernel takes every token and the tiles' second launch,
+  // whose workgroups would all exit, is not made
   constexpr int N = Pack<T>::N;
   if (tokens * kv_heads > INT32_MAX) return fail(NVF_ERR_INVALID, "paged_attention: too many tokens");
   const float sl = scale * 1.4426950408889634f;
@@ -1393,7 +1445,7 @@ int attention_dispatch(const void* q, void* out, const void* kc, const void* vc,
     const int rc = launch_status("paged_attention(tiles)");
     if (rc != NVF_OK) return rc;
   }
-  if (tiles && aligned) {
+  if (tiles && taken) {
     if (!split) return NVF_OK;
     attn_split_combine_kernel<T><<<dim3((unsigned)tokens, (unsigned)q_heads), 256, 0, st>>>(part, ot, tokens,
                                                                                             q_heads, sp.nsplit);
@@ -1579,15 +1631,20 @@ int nvf_paged_attention_seqs_ws(const void* q, void* out, const void* k_cache, c
   if (cu_seqlens_host[0] != 0 || cu_seqlens_host[num_seqs] != tokens)
     return fail(NVF_ERR_INVALID, "nvf_paged_attention_seqs_ws: cu_seqlens must run from 0 to tokens=%lld",
                 (long long)tokens);
-  bool aligned = true;
+  bool taken = true;
+  int64_t tile = -1;  // the tile of the last sequence start inside a tile, and its runs so far
+  int runs = 1;
   for (int s = 1; s <= num_seqs; ++s) {
     if (cu_seqlens_host[s] < cu_seqlens_host[s - 1])
       return fail(NVF_ERR_INVALID, "nvf_paged_attention_seqs_ws: cu_seqlens must not decrease");
-    if (s < num_seqs && cu_seqlens_host[s] % kFaBq != 0) aligned = false;
+    if (s == num_seqs || cu_seqlens_host[s] == cu_seqlens_host[s - 1] || cu_seqlens_host[s] % kFaBq == 0) continue;
+    runs = cu_seqlens_host[s] / kFaBq == tile ? runs + 1 : 2;
+    tile = cu_seqlens_host[s] / kFaBq;
+    if (runs > kFaMaxRuns) taken = false;
   }
   return paged_attention_entry(q, out, k_cache, v_cache, query_seq, query_key_len, block_tables, tokens, q_heads,
                                kv_heads, head_dim, block_size, max_blocks, scale, q_stride, max_query_len, workspace,
-                               workspace_bytes, dtype, stream, aligned);
+                               workspace_bytes, dtype, stream, taken);
 }
 
 int nvf_paged_attention(const void* q, void* out, const void* k_cache, const void* v_cache, const int32_t* query_seq,

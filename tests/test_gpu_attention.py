@@ -593,3 +593,34 @@ def test_paged_attention_token_order_out_of_range_entry(gpu):
     torch.cuda.synchronize()
     keep = [i for i in range(n) if i != 3]
     H.assert_bitexact(H.to_host(out[keep]), H.to_host(ref[keep]), "the named tokens")
+
+
+# Tiles that span sequences: how many runs of one sequence the 128-token tiles hold.
+RUN_CASES = [
+    ([100, 60, 200], 0, False),               # two runs per tile, a tail after it
+    ([16] * 8 + [130], 0, False),             # 8 runs: the most the tile kernel walks
+    ([15] * 9 + [150], 0, False),             # 9 and 10 runs: left to the decode kernel
+    ([127, 1, 128, 64, 63, 2], 3, False),     # runs that end and start on the tile's and the halves' edges
+    ([90, 70, 120], 2500, True),              # the same over split key ranges
+]
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=DT_IDS)
+@pytest.mark.parametrize("ci", range(len(RUN_CASES)))
+def test_paged_attention_tiles_of_several_sequences(gpu, dt, ci):
+    """Against the oracle without the host's packing; with it, the same bits."""
+    lens, prefix, split = RUN_CASES[ci]
+    r = H.rng(900 + 10 * ci + dt)
+    q_heads, kv_heads, hd, bs = 8, 2, 128, 64
+    b = H.make_paged(r, [n + prefix for n in lens], lens, q_heads, kv_heads, hd, bs, dt)
+    exact, vmax = H.oracle_attention(b, q_heads, kv_heads, hd, bs, hd ** -0.5, dt)[1:]
+    args = [H.to_dev(b.q, gpu, dt), H.to_dev(b.k_cache, gpu, dt), H.to_dev(b.v_cache, gpu, dt),
+            H.to_dev(b.query_seq, gpu), H.to_dev(b.query_key_len, gpu), H.to_dev(b.block_tables, gpu)]
+    if split:
+        assert ops.lib().nvf_paged_attention_workspace_size(b.tokens, q_heads, kv_heads, hd, bs, b.max_blocks, 0) > 0
+    case(f"attention runs {lens} prefix={prefix} dt={dt}")
+    got = ops.paged_attention(*args, bs, hd ** -0.5, split=split)
+    assert_attn(H.to_host(got), exact, vmax, dt, f"runs {lens}")
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    host = ops.paged_attention(*args, bs, hd ** -0.5, split=split, cu_seqlens=cu)
+    H.assert_bitexact(H.to_host(host), H.to_host(got), "host cu_seqlens vs device-only metadata")
