@@ -30,6 +30,10 @@ int gemm16(const void* x, const void* w, bool bf16, void* out, int out_dtype, in
 int kq_gemm(const void* x, bool bf16, const void* w, int kind, int layout, void* out, int out_dtype, int64_t m,
             int64_t n, int64_t k, hipStream_t st);
 
+// kq_gemv.hip: K-quant W, m <= 16, x 16-byte aligned, k a multiple of 256
+int kq_gemv(const void* x, int x_dtype, const void* w, int kind, int layout, void* out, int out_dtype, int64_t m,
+            int64_t n, int64_t k, hipStream_t st);
+
 template <typename TO>
 constexpr int dtype_of() {
   return sizeof(TO) == 4 ? NVF_F32 : __is_same(TO, __bf16) ? NVF_BF16 : NVF_F16;
@@ -332,10 +336,32 @@ int launch_dense(const void* x, const Src& src, void* out, int64_t m, int64_t n,
   return launch_status("dense_gemm");
 }
 
+// Where the 16-bit matrix-core decode product of kq_gemv.hip beats the products on decoded
+// weights above.  Q4_K, us (there / here), weights not in the cache:
+//   fp16 x, m =                1            2            4            8            16
+//   151936 x 4096        67 / 136     75 / 155     79 / 247     94 / 249    124 / 254
+//   37888 x 3584       22.5 / 29.5  21.5 / 36.1  23.1 / 58.9  27.2 / 59.2  35.9 / 61.4
+//   4608 x 3584         7.7 / 6.9    8.8 / 8.4   10.2 / 14.3  13.2 / 14.5  19.6 / 15.2
+//   3584 x 18944       14.3 / 17.1  17.3 / 21.6  22.5 / 38.3  32.4 / 38.8  52.1 / 39.2
+//   fp32 x
+//   37888 x 3584       33.3 / 33.1  34.2 / 45.6  37.4 / 54.9  43.8 / 57.3  69.3 / 69.3
+//   4608 x 3584        12.2 / 8.1   12.3 / 11.8  14.9 / 14.1  26.8 / 14.8  41.5 / 19.2
+//   3584 x 18944       25.2 / 20.4  25.7 / 31.4  32.4 / 35.1  68.1 / 36.0
+// (bf16 x: as fp16, a little slower; 1 x 3584 x 18944 18.4 / 17.1).  Narrow outputs have few
+// workgroups over which to spread its staging of x.
+bool kq_gemv_wins(int x_dtype, int64_t m, int64_t n, int64_t k) {
+  if (n >= 16384) return true;
+  if (x_dtype == NVF_F32) return m >= 2 && m <= 4 && k >= 8192;
+  return m <= 8 && (m > 2 || (k >= 8192 && (m == 2 || x_dtype == NVF_F16)));
+}
+
 template <typename TX, typename TO>
 int dispatch_weights(const void* x, const void* w, int w_format, int layout, void* out, int64_t m, int64_t n,
                      int64_t k, bool vec, hipStream_t st) {
   const uint8_t* wb = static_cast<const uint8_t*>(w);
+  if ((w_format == NVF_W_Q4_K || w_format == NVF_W_Q5_K) && vec && m <= kGemvRows && k % 256 == 0 &&
+      k < (1 << 22) && kq_gemv_wins(dtype_of<TX>(), m, n, k))
+    return kq_gemv(x, dtype_of<TX>(), w, w_format, layout, out, dtype_of<TO>(), m, n, k, st);
   if constexpr (sizeof(TX) == 2) {  // whole superblocks per row: the 16-bit matrix cores
     if (w_format >= NVF_W_Q4_K && vec && m > kGemvRows && k % 256 == 0 && k < (1 << 22))
       return kq_gemm(x, __is_same(TX, __bf16), w, w_format, layout, out, dtype_of<TO>(), m, n, k, st);

@@ -81,12 +81,18 @@ def test_non_finite_operands(gpu, dtype):
 
 
 # ---------------------------------------------------------------------------
-# K-quant weights with 16-bit activations (kq_gemm.hip), whole superblocks per row
+# K-quant weights (kq_gemm.hip, and kq_gemv.hip up to 16 rows), whole superblocks per row
 # ---------------------------------------------------------------------------
 KQ = [(12, H.GGML), (12, H.HIP_LEGACY), (13, H.GGML), (14, H.GGML)]
 KQ_IDS = ["q4k", "q4k_legacy", "q5k", "q6k"]
 # the workgroup's rows beside each
 KQ_SIZES = [
+    (1, 16400, 256),     # decode: one row, one superblock, 16 of 64 columns in the last workgroup
+    (3, 100, 512),       # 8 K groups, most of them without a superblock
+    (5, 33, 2304),       # two results per lane, one column past whole wave groups
+    (8, 16390, 768),     # x in one stage
+    (13, 16400, 2304),   # x in several stages, all four results per lane
+    (2, 40, 8192),       # narrow and deep
     (17, 130, 256),      # 32: one superblock, two columns in the last tile
     (33, 129, 2304),     # 64
     (65, 24577, 256),    # 128
@@ -106,9 +112,11 @@ def kq_oracle(x, dt, w, kind, layout, m, n, k):
 
 
 @pytest.mark.parametrize("kind,layout", KQ, ids=KQ_IDS)
-@pytest.mark.parametrize("dt", [H.F16, H.BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("dt", [H.F16, H.BF16, H.F32], ids=["f16", "bf16", "f32"])
 @pytest.mark.parametrize("m,n,k", KQ_SIZES)
 def test_kquant_within_fp32_sum_bound(gpu, kind, layout, dt, m, n, k):
+    if dt == H.F32 and m > 16:
+        pytest.skip("fp32 rows beyond the decode product take the tile kernel of test_gpu_dense_gemm.py")
     print(f"[case] kq {kind}/{layout} {m}x{n}x{k} dt={dt}", flush=True)
     x, w = kq_case(100 * kind + m, m, n, k, dt, kind)
     want, err = kq_oracle(x, dt, w, kind, layout, m, n, k)
@@ -125,13 +133,14 @@ def test_kquant_within_fp32_sum_bound(gpu, kind, layout, dt, m, n, k):
 
 @pytest.mark.parametrize("kind,layout", KQ, ids=KQ_IDS)
 @pytest.mark.parametrize("dt", [H.F16, H.BF16], ids=["f16", "bf16"])
-def test_kquant_non_finite_operands(gpu, kind, layout, dt):
-    m, n, k = 40, 150, 512
+@pytest.mark.parametrize("m", [40, 7], ids=["prefill", "decode"])
+def test_kquant_non_finite_operands(gpu, kind, layout, dt, m):
+    n, k = 150, 512
     x, w = kq_case(7 * kind, m, n, k, dt, kind)
     xt = H.to_dev(x, gpu, dt)
-    xt[3, 7], xt[9, 300], xt[20, 0] = float("inf"), float("-inf"), float("nan")
+    xt[3, 7], xt[5, 300], xt[1, 0] = float("inf"), float("-inf"), float("nan")
     if dt == H.BF16:
-        xt[30, 5] = 3.0e38  # finite, but not times a sub-block's whole-number scale
+        xt[6, 5] = 3.0e38  # finite, but not times a sub-block's whole-number scale
     blk = w.reshape(n * k // 256, -1)
     d_at = 208 if kind == 14 else 0
     blk[4 * 2 + 1, d_at:d_at + 2] = np.array([np.inf], np.float16).view(np.uint8)  # column 4's second superblock
