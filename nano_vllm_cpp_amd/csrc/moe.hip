@@ -8,18 +8,21 @@
 // workgroup per token for the FFN, with a scalar dot product per weight row.
 //
 // Routing (moe_route_kernel): one wave per row, the reference's arithmetic in
-// double in its order -- the maximum and the sums by one lane in index order, the
+// double in its order -- the sums by one lane in index order, the maximum and the
 // exponentials in parallel, and the top-K selection as the reference's selection
 // sort: each round takes the largest value at positions >= i (a tie goes to the
 // smallest position: its strict-greater scan) and swaps it to position i.  So the
 // experts chosen and their order, ties included, are the reference's, and the
-// scores are its doubles rounded once to fp32.  (NaN logits are outside this: the
+// scores are its doubles rounded once to fp32.  (256 rows x 128 experts, top 8: 19.1 us with
+// the maximum in one lane and the rounds' reductions through LDS permutes, 9.3 with both by
+// DPP.)  (NaN logits are outside this: the
 // reference's result then depends on its scan order.)
 //
 // Expert FFN: out[t] += sum_k w[t,k] * down_e(silu(gate_e(x[t])) * up_e(x[t])),
 // e = slot_of[idx[t,k]], for w != 0.  On the GPU the (token, k) pairs are grouped by
-// expert slot, and each slot's pairs run as one matrix product on the fp32 matrix
-// cores (the tile kernel of gemm_tile.hpp with a gathering problem policy):
+// expert slot, and each slot's pairs run as one matrix product (bf16 weights:
+// moe16_kernel below, with steps 3 and 4 in one; else the tile kernel of gemm_tile.hpp
+// on the fp32 matrix cores, with a gathering problem policy):
 //   1. count the pairs per slot, scan, and list each slot's 32- or 128-row tiles;
 //   2. scatter the pairs into slot order;
 //   3. gate/up: [pairs of slot s] x gu[s]^T -> GU (fp32, 2I per pair);
@@ -32,12 +35,32 @@
 // results agree within the bound the tests state, not bit for bit.
 #include <mutex>
 
+#include "gemm16.hpp"
 #include "gemm_tile.hpp"
 
 namespace nvf {
 
 // ---------------------------------------------------------------------------
 // routing
+
+// The largest of the wave's values, in every lane: DPP inside 16 lanes, a swizzle across
+// them, and the two halves (as group_max).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double wave_max_f64(double v) {
+  v = fmax(v, dpp_f64<0xb1>(v));
+  v = fmax(v, dpp_f64<0x4e>(v));
+  v = fmax(v, dpp_f64<0x141>(v));
+  v = fmax(v, dpp_f64<0x140>(v));
+  v = fmax(v, __shfl_xor(v, 16, 64));
+  return fmax(v, __shfl_xor(v, 32, 64));
+}
+
 constexpr int kMoeMaxExperts = 4096;
 
 __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__ logits, int E, int K, int norm,
@@ -45,24 +68,22 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
   extern __shared__ __attribute__((aligned(16))) double rsm[];
   double* pr = rsm;                                   // [E] values, permuted by the selection
   int* ix = reinterpret_cast<int*>(rsm + E);          // [E] expert ids, permuted alike
-  __shared__ double s_max, s_inv;
+  __shared__ double s_inv;
   const int64_t t = blockIdx.x;
   const int lane = threadIdx.x;
   const float* lg = logits + t * E;
-  if (lane == 0) {  // the reference's running maximum, in index order
-    double m = -1e300;
-    for (int i = 0; i < E; ++i) {
-      const double v = (double)lg[i];
-      m = m > v ? m : v;
-    }
-    s_max = m;
+  // the reference's running maximum (a maximum does not depend on the order)
+  double m = -1e300;
+  for (int i = lane; i < E; i += 64) {
+    const double v = (double)lg[i];
+    m = m > v ? m : v;
   }
-  __syncthreads();
-  const double maxv = s_max;
+  const double maxv = wave_max_f64(m);
   for (int i = lane; i < E; i += 64) pr[i] = exp((double)lg[i] - maxv);
   __syncthreads();
   if (lane == 0) {
     double sum = 0.0;
+#pragma unroll 16
     for (int i = 0; i < E; ++i) sum += pr[i];
     s_inv = 1.0 / sum;
   }
@@ -84,15 +105,16 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
         bv = pr[j];
         bp = j;
       }
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-      const double ov = __shfl_xor(bv, d, 64);
-      const int op = __shfl_xor(bp, d, 64);
-      if (ov > bv || (ov == bv && op < bp)) {
-        bv = ov;
-        bp = op;
-      }
+    // the wave's largest, and the smallest of the positions that hold it (a NaN at
+    // position i is every lane's value and equals none: position i stays)
+    const double best = wave_max_f64(bv);
+    uint64_t eq = __ballot(bv == best);
+    int pos = eq ? INT32_MAX : i;
+    for (; eq; eq &= eq - 1) {
+      const int q = __builtin_amdgcn_readlane(bp, __builtin_ctzll(eq));
+      pos = q < pos ? q : pos;
     }
+    bp = pos;
     if (lane == 0) {
       const double tp = pr[i];
       pr[i] = pr[bp];
@@ -255,6 +277,68 @@ __global__ void moe_scatter_kernel(const int32_t* __restrict__ idx, const float*
   for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < pairs; p += (int64_t)gridDim.x * blockDim.x) {
     const int s = pair_slot(idx, score, slot_of, p, slots);
     if (s >= 0) list[offsets[s] + atomicAdd(cursor + s, 1)] = (int32_t)p;
+  }
+}
+
+// The same grouping by one workgroup, with the counts in LDS (slots <= kGroupSlots).
+constexpr int kGroupMax = 4096;
+__global__ __launch_bounds__(kScanThreads) void moe_group_kernel(
+    const int32_t* __restrict__ idx, const float* __restrict__ score, const int32_t* __restrict__ slot_of, int pairs,
+    int slots, int bm, int32_t* __restrict__ list, int32_t* __restrict__ tile_slot, int32_t* __restrict__ tile_pos,
+    int32_t* __restrict__ tile_end, int32_t* __restrict__ ntiles) {
+  __shared__ int32_t at[kGroupMax], part_rows[kScanThreads / 64], part_tiles[kScanThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int s = tid; s < slots; s += kScanThreads) at[s] = 0;
+  __syncthreads();
+  for (int p = tid; p < pairs; p += kScanThreads) {
+    const int s = pair_slot(idx, score, slot_of, p, slots);
+    if (s >= 0) atomicAdd(at + s, 1);
+  }
+  __syncthreads();
+  // exclusive scans over the slots (thread t: slots [t per, +per)): lanes, then waves
+  const int per = (slots + kScanThreads - 1) / kScanThreads;
+  const int s0 = tid * per < slots ? tid * per : slots, s1 = s0 + per < slots ? s0 + per : slots;
+  int rows = 0, tiles = 0;
+  for (int s = s0; s < s1; ++s) {
+    rows += at[s];
+    tiles += (at[s] + bm - 1) / bm;
+  }
+  int r = rows, tl = tiles;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int a = __shfl_up(r, d), b = __shfl_up(tl, d);
+    if (lane >= d) {
+      r += a;
+      tl += b;
+    }
+  }
+  if (lane == 63) {
+    part_rows[wave] = r;
+    part_tiles[wave] = tl;
+  }
+  r -= rows;
+  tl -= tiles;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) {
+    r += part_rows[w];
+    tl += part_tiles[w];
+  }
+  if (tid == kScanThreads - 1) *ntiles = tl + tiles;
+  for (int s = s0; s < s1; ++s) {
+    const int c = at[s];
+    at[s] = r;  // the slot's next free row
+    for (int i = 0; i < c; i += bm) {
+      tile_slot[tl] = s;
+      tile_pos[tl] = r + i;
+      tile_end[tl] = r + c;
+      ++tl;
+    }
+    r += c;
+  }
+  __syncthreads();
+  for (int p = tid; p < pairs; p += kScanThreads) {
+    const int s = pair_slot(idx, score, slot_of, p, slots);
+    if (s >= 0) list[atomicAdd(at + s, 1)] = p;
   }
 }
 
@@ -426,18 +510,218 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restric
   }
 }
 
-// How a call runs: up to 4096 pairs are grouped by the one-launch sort, more by
-// counting; rows per expert tile are 16 on the decode product (the grouped form of
-// the weight-streaming GEMV, when rows are whole 8-element runs and aligned), else
+// ---------------------------------------------------------------------------
+// bf16 expert weights: both products on the bf16 matrix cores as gemm16_kernel runs them
+// (both operands HBM -> LDS by DMA, K in 64-value stages), over the same tiles and
+// with the rows gathered by the DMA's per-lane addresses.  Activations are XP exact bf16
+// planes: bf16 x as it is, fp16 and fp32 x split beforehand (2 and 3 planes), and the
+// SwiGLU rows as three planes written by the gate/up product's own epilogue, which
+// takes gate and up columns of the same index into one tile (so GU and its fp32 Y
+// never reach memory).
+//
+// Bound by the expert weights' stream at decode batches: 256 rows, 128 experts of 768
+// (H 2048), top 8: gate/up 237 us (805 MB) and down 144 us (403 MB) on gemv_mfma_kernel,
+// whose 16-row tiles gather their rows for every 64 columns and load step by step; here 165
+// (4.9 TB/s) and 90.  Tiles of 32 rows x 128 columns with four stages in the ring (two for
+// three planes) measured best: 64 columns in 2 K groups 172 and 104, 256 columns 195 and
+// 93, five stages 173, 128 columns by two waves 168.
+
+// x [rows][H] -> planes [XP][rows][H], 8 values per thread.
+template <typename TX, int XP>
+__global__ __launch_bounds__(256) void moe_split_kernel(const TX* __restrict__ x, int64_t n8, __bf16* __restrict__ p) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n8) return;
+  const Table<8, TX> xs{x};
+  float v[8];
+  xs.decode(xs.load(i * 8), v);
+  bf16x8 pc[3];
+  split3(v, pc);
+#pragma unroll
+  for (int q = 0; q < XP; ++q) st16(p + (q * n8 + i) * 8, __builtin_bit_cast(u32x4, pc[q]));
+}
+
+// One product over the expert tiles.  GU: columns [0, BN / 2) of a tile are gate rows and the
+// rest the up rows of the same indices of w [2 I][k]; the epilogue writes the SwiGLU planes
+// yp [3][list rows][I].  Else: w [n_cols][k], results to v_out [pair][n_cols].
+template <bool GU, int XP, int BM, int BN, int WM, int WN, int KG, int NS, int OCC>
+__global__ __launch_bounds__(WM* WN* KG * 64) __attribute__((amdgpu_waves_per_eu(OCC))) void moe16_kernel(
+    const __bf16* __restrict__ xp, int64_t plane, int64_t x_per, const __bf16* __restrict__ w, MoeTiles prob, int64_t k,
+    __bf16* __restrict__ yp, int64_t yplane, float* __restrict__ v_out) {
+  constexpr int BK = 64, kWaves = WM * WN, TM = BM / WM / 32, TN = BN / WN / 32;
+  constexpr int kRowB = BK * 2, kRows = XP * BM + BN, kStage = kRows * kRowB;
+  constexpr int kDma = kStage / 1024 / kWaves;
+  static_assert(kStage % (1024 * kWaves) == 0, "stage transfers");
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave_id = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int group = KG == 1 ? 0 : wave_id / kWaves, wave = KG == 1 ? wave_id : wave_id % kWaves;
+  const int wm = wave / WN, wn = wave % WN;
+  uint8_t* const ring = lds + group * (NS * kStage);
+  const int half = lane >> 5, lr = lane & 31;
+  const int ar = wm * TM * 32 + lr, br = XP * BM + wn * TN * 32 + lr;
+  const int a0 = ar * kRowB + ((half ^ g16_key<BK>(ar)) << 4);
+  const int b0 = br * kRowB + ((half ^ g16_key<BK>(br)) << 4);
+  const int64_t n = GU ? 2 * prob.n_cols : prob.n_cols;  // weight rows per slot (GU: n_cols = I columns, BN / 2 per tile)
+  const int nst = (int)((k + BK - 1) / BK), steps = (nst + KG - 1) / KG;
+
+  for (int64_t item = blockIdx.x;; item += gridDim.x) {
+    MoeTiles::Tile t;
+    if (!prob.pick(item, t)) break;  // uniform per workgroup
+    const __bf16* wbase = w + t.slot * n * k;
+    const __amdgpu_buffer_rsrc_t rw = g16_rsrc(wbase, n * k * 2);
+    // this lane's 16-byte chunk of each transfer: a row past the tile's, or a column past
+    // n_cols, reads zero
+    uint32_t off[kDma];
+    int kchunk[kDma];
+#pragma unroll
+    for (int i = 0; i < kDma; ++i) {
+      const int r = (wave * kDma + i) * 8 + (lane >> 3), c = (lane & 7) ^ g16_key<BK>(r);
+      kchunk[i] = c * 8;
+      if (r < XP * BM) {
+        const int64_t pos = t.pos0 + r % BM;
+        const bool ok = pos < t.pos_end;
+        const int64_t row = ok ? (GU ? (int64_t)prob.list[pos] / x_per : pos) : 0;
+        off[i] = ok ? (uint32_t)((row * k + c * 8) * 2) : 0x80000000u;
+      } else {
+        const int col = r - XP * BM;
+        const int64_t cc = t.col0 + (GU ? col % (BN / 2) : col);
+        const int64_t wr = GU && col >= BN / 2 ? prob.n_cols + cc : cc;
+        off[i] = cc < prob.n_cols ? (uint32_t)((wr * k + c * 8) * 2) : 0x80000000u;
+      }
+    }
+    auto issue = [&](int step, int buf) {
+      const int st = step * KG + group;
+      const bool tail = (int64_t)(st + 1) * BK > k;
+#pragma unroll
+      for (int i = 0; i < kDma; ++i) {
+        const int r8 = (wave * kDma + i) * 8;  // uniform: BM and BN are multiples of 8
+        uint32_t o = off[i];
+        if (tail) o = (int64_t)st * BK + kchunk[i] < k ? o : 0x80000000u;
+        const __amdgpu_buffer_rsrc_t ra = g16_rsrc(xp + (r8 < XP * BM ? r8 / BM : 0) * plane, plane * 2);
+        g16_dma(r8 < XP * BM ? ra : rw, ring + buf * kStage + (wave * kDma + i) * 1024, o, (uint32_t)st * kRowB);
+      }
+    };
+
+    f32x16 acc[TN][TM];
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+      for (int b = 0; b < TM; ++b) acc[a][b] = f32x16{};
+#pragma unroll
+    for (int s = 0; s < NS - 1; ++s) issue(s, s);
+    int buf = 0;
+#pragma unroll 1
+    for (int st = 0; st < steps; ++st) {
+      wait_vm<(NS - 2) * kDma>();
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      issue(st + NS - 1, buf == 0 ? NS - 1 : buf - 1);
+      const uint8_t* s = ring + buf * kStage;
+#pragma unroll
+      for (int kk = 0; kk < BK / 16; ++kk) {
+        u32x4 wb[TN];
+#pragma unroll
+        for (int a = 0; a < TN; ++a) wb[a] = ld16(s + (b0 ^ (kk << 5)) + a * 32 * kRowB);
+#pragma unroll
+        for (int p = XP - 1; p >= 0; --p)  // the smallest pieces first
+#pragma unroll
+          for (int b = 0; b < TM; ++b) {
+            const u32x4 xa = ld16(s + p * BM * kRowB + (a0 ^ (kk << 5)) + b * 32 * kRowB);
+#pragma unroll
+            for (int a = 0; a < TN; ++a) acc[a][b] = mfma16(wb[a], xa, acc[a][b], __bf16{});
+          }
+      }
+      buf = buf == NS - 1 ? 0 : buf + 1;
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this stage's reads are done before the barrier
+    }
+    wait_vm<0>();
+    __syncthreads();
+
+    // the tile in LDS as fp32 [BM][BN], the K groups adding their sums in group order
+    constexpr int kPitch = BN * 4 + 16;
+#pragma unroll 1
+    for (int g = 0; g < KG; ++g) {
+      if (group == g) {
+#pragma unroll
+        for (int b = 0; b < TM; ++b)
+#pragma unroll
+          for (int a = 0; a < TN; ++a)
+#pragma unroll
+            for (int jq = 0; jq < 4; ++jq) {
+              uint8_t* d = lds + (wm * TM * 32 + 32 * b + lr) * kPitch + (wn * TN * 32 + 32 * a + 8 * jq + 4 * half) * 4;
+              float v[4];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[e] = acc[a][b][4 * jq + e];
+              if (g > 0) {
+                float o[4];
+                Pack<float>::unpack(ld16(d), o);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] += o[e];
+              }
+              st16(d, Pack<float>::pack(v));
+            }
+      }
+      __syncthreads();
+    }
+    constexpr int kThreads = kWaves * KG * 64;
+    if constexpr (GU) {
+      constexpr int kVpr = BN / 2 / 8;
+      for (int u = threadIdx.x; u < BM * kVpr; u += kThreads) {
+        const int r = u / kVpr, c = (u % kVpr) * 8;
+        const int64_t pos = t.pos0 + r, col = t.col0 + c;
+        if (pos >= t.pos_end || col >= prob.n_cols) continue;
+        float gate[8], up[8], y[8];
+        const uint8_t* d = lds + r * kPitch + c * 4;
+        Pack<float>::unpack(ld16(d), gate);
+        Pack<float>::unpack(ld16(d + 16), gate + 4);
+        Pack<float>::unpack(ld16(d + BN * 2), up);
+        Pack<float>::unpack(ld16(d + BN * 2 + 16), up + 4);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = silu_mul<float>(gate[e], up[e]);
+        bf16x8 pc[3];
+        split3(y, pc);
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          st16(yp + q * yplane + pos * prob.n_cols + col, __builtin_bit_cast(u32x4, pc[q]));
+      }
+    } else {
+      constexpr int kVpr = BN / 4;
+      for (int u = threadIdx.x; u < BM * kVpr; u += kThreads) {
+        const int r = u / kVpr, c = (u % kVpr) * 4;
+        const int64_t pos = t.pos0 + r, col = t.col0 + c;
+        if (pos < t.pos_end && col < prob.n_cols)
+          st16(v_out + (int64_t)prob.list[pos] * prob.n_cols + col, ld16(lds + r * kPitch + c * 4));
+      }
+    }
+    __syncthreads();  // LDS is reused by the next item
+  }
+}
+
+// How a call runs.  Grouping: one workgroup counting in LDS, up to kGroupSlots slots and
+// kGroupPairs pairs (256 rows x top 8: 19 us in four launches -> 5.8); else the one-launch
+// sort, up to 4096 pairs (the drop-in, which does not know its slots); else four launches.
+// Products with bf16 weights: moe16_kernel over tiles of 32, 64 or 128 rows by the pairs per
+// expert that a call brings; the FFN of Qwen3-30B-A3B's experts on bf16 x, us, from the
+// products below: 2 rows 51 -> 43, 16 rows 204 -> 182, 256 rows 389 -> 268, 1024 rows 590 -> 406,
+// 4096 rows 1465 -> 1047 (fp32 x: 53 -> 48, 233 -> 211, 429 -> 304, 610 -> 507, 1592 -> 1479).
+// Below 16 pairs its tiles are 64 columns wide, to have enough of them (one row, bf16
+// x: 33 us against 37, and 35 below); there fp16 and fp32 x gain nothing over the products
+// below.
+// fp16 weights, or unaligned rows: 16 rows per expert tile on the decode product (the grouped
+// form of the weight-streaming GEMV, when rows are whole 8-element runs and aligned), else
 // 32 or 128 on the tile kernel.
+constexpr int kGroupSlots = kGroupMax, kGroupPairs = 16384;
 struct MoePlan {
-  bool sort, gemv;
+  bool group, sort, gemv, mfma16, few;
   int bm, gemv_c;
-  MoePlan(int64_t pairs, int64_t slots, bool vec_rows) {
-    gemv = pairs <= kSortMax && vec_rows;
-    // the one-launch sort for few pairs, or when counting would scan too many slots
-    sort = pairs <= kSortMax && (pairs <= 512 || slots > kSortMax);
-    bm = gemv ? 16 : pairs >= 4096 ? 128 : 32;
+  MoePlan(int64_t pairs, int64_t slots, bool vec_rows, bool bf16_fits, int planes) {
+    few = pairs < 16;
+    mfma16 = bf16_fits && vec_rows && (planes == 1 || !few);
+    gemv = !mfma16 && pairs <= kSortMax && vec_rows;
+    group = slots <= kGroupSlots && pairs <= kGroupPairs;
+    sort = !group && pairs <= kSortMax;
+    bm = mfma16 ? (pairs >= 16384 ? 128 : pairs >= 4096 ? 64 : 32) : gemv ? 16 : pairs >= 4096 ? 128 : 32;
     // 64 columns per workgroup once there are enough tiles: each workgroup gathers its
     // tile's activation rows once for 4x the weight columns
     gemv_c = pairs >= 256 ? 4 : 1;
@@ -483,13 +767,46 @@ int moe_product(const TX* a, const TW* w, Prob prob, int64_t k, const MoePlan& p
   return launch_status("moe expert product");
 }
 
+// One of the two products of the bf16 path.
+template <bool GU, int XP, int BM, int BN, int WM, int WN, int KG, int NS, int OCC>
+int launch_moe16(const __bf16* xp, int64_t plane, int64_t x_per, const __bf16* w, MoeTiles prob, int64_t k, __bf16* yp,
+                 int64_t yplane, float* v, int64_t max_tiles, hipStream_t st) {
+  constexpr int kRing = KG * NS * (XP * BM + BN) * 128, kEpi = BM * (BN * 4 + 16), kLds = kRing > kEpi ? kRing : kEpi;
+  auto kern = moe16_kernel<GU, XP, BM, BN, WM, WN, KG, NS, OCC>;
+  static std::once_flag attr_once;
+  std::call_once(attr_once, [&] {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+  });
+  prob.cols = GU ? BN / 2 : BN;
+  kern<<<moe_grid(max_tiles, (prob.n_cols + prob.cols - 1) / prob.cols), WM * WN * KG * 64, kLds, st>>>(
+      xp, plane, x_per, w, prob, k, yp, yplane, v);
+  return launch_status("moe expert product (bf16)");
+}
+template <bool GU, int XP>
+int moe_product16(const __bf16* xp, int64_t plane, int64_t x_per, const __bf16* w, const MoeTiles& prob, int64_t k,
+                  __bf16* yp, int64_t yplane, float* v, const MoePlan& plan, int64_t max_tiles, hipStream_t st) {
+  if (plan.bm == 128)
+    return launch_moe16<GU, XP, 128, 128, 4, 2, 1, 2, 2>(xp, plane, x_per, w, prob, k, yp, yplane, v, max_tiles, st);
+  if (plan.bm == 64)
+    return launch_moe16<GU, XP, 64, 128, 2, 2, 1, 2, 2>(xp, plane, x_per, w, prob, k, yp, yplane, v, max_tiles, st);
+  if (plan.few)
+    return launch_moe16<GU, XP, 32, 64, 1, 2, 2, 2, 2>(xp, plane, x_per, w, prob, k, yp, yplane, v, max_tiles, st);
+  return launch_moe16<GU, XP, 32, 128, 1, 4, 1, XP == 1 ? 4 : 2, 2>(xp, plane, x_per, w, prob, k, yp, yplane, v,
+                                                                    max_tiles, st);
+}
+
 template <typename TX, typename TW>
 int launch_moe_ffn(const TX* x, const int32_t* idx, const float* score, const TW* gu, const TW* dn,
                    const int32_t* slot_of, int64_t rows, int64_t H, int64_t I, int64_t K, int64_t slots, void* out,
                    int out_dtype, uint8_t* work, hipStream_t st) {
   const int64_t pairs = rows * K;
   const bool aligned = aligned16(x) && aligned16(gu) && aligned16(dn);
-  const MoePlan plan(pairs, slots, aligned && H % 8 == 0 && I % 8 == 0);
+  // The bf16 path keeps x's planes in V's region (free until the down product) and addresses
+  // its operands with 31-bit offsets.
+  constexpr int XP = __is_same(TX, __bf16) ? 1 : __is_same(TX, _Float16) ? 2 : 3;
+  const bool fits = __is_same(TW, __bf16) && (XP == 1 || XP * rows <= 2 * pairs) && rows * H < (1 << 29) &&
+                    pairs * I < (1 << 29) && 2 * I * H < (1 << 29);
+  const MoePlan plan(pairs, slots, aligned && H % 8 == 0 && I % 8 == 0, fits, XP);
   const bool vec = aligned && H % kDgKC == 0 && I % kDgKC == 0;  // the tile kernel's vector staging
   const MoeLayout L(pairs, H, I, slots, plan.bm);
   int32_t* counts = reinterpret_cast<int32_t*>(work + L.counts);
@@ -503,7 +820,10 @@ int launch_moe_ffn(const TX* x, const int32_t* idx, const float* score, const TW
   float* gu_rows = reinterpret_cast<float*>(work + L.gu);
   float* y_rows = reinterpret_cast<float*>(work + L.y);
   float* v_rows = reinterpret_cast<float*>(work + L.v);
-  if (plan.sort) {
+  if (plan.group) {
+    moe_group_kernel<<<1, kScanThreads, 0, st>>>(idx, score, slot_of, (int)pairs, (int)slots, plan.bm, list, tile_slot,
+                                                 tile_pos, tile_end, ntiles);
+  } else if (plan.sort) {
     int n2 = 1;
     while (n2 < pairs) n2 <<= 1;
     moe_sort_small_kernel<<<1, 1024, 0, st>>>(idx, score, slot_of, (int)pairs, n2, slots, plan.bm, list, tile_slot,
@@ -521,6 +841,31 @@ int launch_moe_ffn(const TX* x, const int32_t* idx, const float* score, const TW
   if (rc != NVF_OK) return rc;
 
   const MoeTiles base{tile_slot, tile_pos, tile_end, ntiles, list, 0, 0};
+  if constexpr (__is_same(TW, __bf16)) {
+    if (plan.mfma16) {
+      const __bf16* xp = reinterpret_cast<const __bf16*>(x);
+      if constexpr (XP > 1) {
+        __bf16* planes = reinterpret_cast<__bf16*>(v_rows);
+        const int64_t n8 = rows * H / 8;
+        moe_split_kernel<TX, XP><<<(unsigned)((n8 + 255) / 256), 256, 0, st>>>(x, n8, planes);
+        rc = launch_status("moe split");
+        if (rc != NVF_OK) return rc;
+        xp = planes;
+      }
+      __bf16* yp = reinterpret_cast<__bf16*>(gu_rows);  // 6 of GU's 8 bytes per value
+      MoeTiles prob = base;
+      prob.n_cols = I;
+      rc = moe_product16<true, XP>(xp, rows * H, K, gu, prob, H, yp, pairs * I, nullptr, plan, L.max_tiles, st);
+      if (rc != NVF_OK) return rc;
+      prob.n_cols = H;
+      rc = moe_product16<false, 3>(yp, pairs * I, 1, dn, prob, I, nullptr, 0, v_rows, plan, L.max_tiles, st);
+      if (rc != NVF_OK) return rc;
+      NVF_DISPATCH_DTYPE(out_dtype, TO,
+                         (moe_combine_kernel<TO><<<(unsigned)rows, 256, 0, st>>>(v_rows, idx, score, slot_of, K, H,
+                                                                                  slots, static_cast<TO*>(out))));
+      return launch_status("moe combine");
+    }
+  }
   {
     MoeGateUp prob;
     static_cast<MoeTiles&>(prob) = base;

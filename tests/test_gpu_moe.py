@@ -244,3 +244,27 @@ def test_add_inplace_and_scale_rows_sigmoid(gpu, ref):
         H.assert_bitexact(mine.cpu().numpy(), theirs.cpu().numpy(), "scale_rows_sigmoid vs reference kernel")
         want = dst * (1.0 / (1.0 + np.exp(-s.astype(np.float64))))[:, None]
         assert np.allclose(mine.cpu().numpy(), want, rtol=4 * 2 ** -24, atol=0)
+
+
+@pytest.mark.parametrize("x_dt", DTYPES, ids=DT_IDS)
+@pytest.mark.parametrize("rows,hid,inter,k,n_exp,slots", [
+    (2, 136, 40, 7, 7, 7),           # 14 pairs: the 64-column tiles
+    (2, 136, 40, 8, 8, 8),           # 16 pairs: the 128-column tiles, K over two stages
+    (512, 72, 136, 8, 20, 4096),     # 4096 pairs: 64-row tiles; the most slots counted in LDS
+    (520, 200, 24, 8, 16, 4097),     # one slot more: the launches of their own
+    (2048, 64, 72, 8, 9, 12),        # 16384 pairs: 128-row tiles; the most pairs counted in LDS
+    (2049, 64, 24, 8, 130, 130),     # eight pairs more, most tiles of a few rows
+])
+def test_moe_ffn_bf16_tiles(gpu, x_dt, rows, hid, inter, k, n_exp, slots):
+    """Every tile shape and grouping of the bf16 weights' path, at sizes that are not whole
+    tiles or stages, with skipped pairs."""
+    r = H.rng(rows + hid + x_dt)
+    x, gu, dn, idx, score, slot_of = moe_case(r, rows, hid, inter, k, n_exp, slots, True, x_dt)
+    score[0, -1] = 0.0
+    slot_of[idx[1, 0]] = -1
+    out_in = H.gen_act(r, (rows, hid), H.F32)
+    ideal, err = oracle_ffn(x, x_dt, gu, dn, True, idx, score, slot_of, slots, H.from_storage(out_in, H.F32))
+    case(f"nvf_moe_ffn bf16 tiles x={x_dt} rows={rows} H={hid} I={inter} K={k} slots={slots}")
+    got = ops.moe_ffn(H.to_dev(x, gpu, x_dt), H.to_dev(idx, gpu), H.to_dev(score, gpu), H.to_dev(gu, gpu, H.BF16),
+                      H.to_dev(dn, gpu, H.BF16), H.to_dev(slot_of, gpu), inter, slots, H.to_dev(out_in, gpu, H.F32))
+    assert_within(H.to_host(got), ideal, err, H.F32, "moe_ffn bf16 tiles", True)
