@@ -116,6 +116,8 @@ class NvfError(RuntimeError):
 def lib() -> C.CDLL:
     """Loads libnvf_ops.so once; raises if it has not been built."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is None:
             if not LIB_PATH.exists():
@@ -138,7 +140,10 @@ def _check(status: int, what: str) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # torch.cuda.current_stream().cuda_stream without the Stream object: 0.2 us against 2.7,
+    # of the 9 to 12 us that a small call spends on the host (a tensor on the GPU, and so an
+    # initialized torch.cuda, is there by now: the pointers are taken first)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dev(t: torch.Tensor, name: str) -> int:
@@ -154,8 +159,10 @@ def _dev_rows(t: torch.Tensor, name: str) -> int:
     remaining dimensions are contiguous within a row."""
     if not t.is_cuda:
         raise ValueError(f"{name} must be a GPU tensor")
-    if not t[0:1].reshape(-1).is_contiguous() or t.stride(-1) != 1 or \
-            (t.dim() > 2 and t.stride(-2) != t.shape[-1]):
+    dim = t.dim()
+    # up to three dimensions the strides alone say that a row is contiguous
+    if t.stride(-1) != 1 or (dim > 2 and t.stride(-2) != t.shape[-1]) or \
+            (dim > 3 and not t[0:1].reshape(-1).is_contiguous()):
         raise ValueError(f"{name} must have contiguous rows")
     return t.data_ptr()
 
