@@ -14,7 +14,7 @@
 // leaves only the fp32 matrix cores, 16 times slower.
 //
 // 1021 x 37888 x 3584, fp16 x, Q4_K: the fp32 matrix-core tile kernel takes 2487 us (111
-// TFLOP/s).  Activations reach LDS by DMA; a weight stage is loaded to registers two
+// TFLOP/s), this one 430 (645).  Activations reach LDS by DMA; a weight stage is loaded to registers two
 // stages ahead, decoded once per workgroup and stored to LDS as 16-bit operands.
 //
 // Infinities and NaN: x and P are multiplied apart from the weight's scale and offset, so a
