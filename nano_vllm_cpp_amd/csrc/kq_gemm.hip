@@ -14,7 +14,8 @@
 // leaves only the fp32 matrix cores, 16 times slower.
 //
 // 1021 x 37888 x 3584, fp16 x, Q4_K: the fp32 matrix-core tile kernel takes 2487 us (111
-// TFLOP/s), this one 430 (645).  Activations reach LDS by DMA; a weight stage is loaded to registers two
+// TFLOP/s), this one 406 (683; 430 with the
+// headers read in every stage, the loads left behind the products and B set to 0 by moves).  Activations reach LDS by DMA; a weight stage is loaded to registers two
 // stages ahead, decoded once per workgroup and stored to LDS as 16-bit operands.
 //
 // Infinities and NaN: x and P are multiplied apart from the weight's scale and offset, so a
@@ -32,18 +33,21 @@ namespace nvf {
 
 constexpr int kKqBN = 128, kKqBK = 64;
 
-// One stage of one thread: NB bytes of quants of column c, part p of its 64 K values (and
-// the superblock header).  put() hands (chunk, 8 integers q as bytes, scale index) on.
+// One stage of one thread: NB bytes of quants of column c, part p of its 64 K values.  Head is
+// what a superblock's four stages share, loaded once for them: read again in every
+// stage, the compiler merges it with the older copy and waits for the newest load.  put() hands (chunk, 8 integers q as bytes, scale index) on.
 template <int KIND, int LAYOUT, int NB>
 struct KqRaw;
 
 template <int LAYOUT, int NB>
 struct KqRaw<NVF_Q4_K, LAYOUT, NB> {
   static constexpr int kBlock = 144;
-  u32x4 hdr;
+  struct Head {
+    u32x4 w;
+    __device__ __forceinline__ void load(const uint8_t* blk, int) { w = ld16(blk); }
+  } hd;
   uint32_t q[NB / 4];
   __device__ __forceinline__ void load(const uint8_t* blk, int quarter, int part) {
-    hdr = ld16(blk);
     const uint8_t* p = blk + 16 + 32 * quarter + NB * part;
     if constexpr (NB == 16) {
       const u32x4 v = ld16(p);
@@ -70,34 +74,43 @@ struct KqRaw<NVF_Q4_K, LAYOUT, NB> {
     }
   }
   __device__ __forceinline__ void scale_min(int j, uint32_t& sc, uint32_t& mn) const {
-    q4k_sm(hdr[1], hdr[2], hdr[3], j, sc, mn);
+    q4k_sm(hd.w[1], hd.w[2], hd.w[3], j, sc, mn);
   }
-  __device__ __forceinline__ float d() const { return half_bits_to_f32(hdr[0] & 0xffffu); }
-  __device__ __forceinline__ float dmin() const { return half_bits_to_f32(hdr[0] >> 16); }
+  __device__ __forceinline__ float d() const { return half_bits_to_f32(hd.w[0] & 0xffffu); }
+  __device__ __forceinline__ float dmin() const { return half_bits_to_f32(hd.w[0] >> 16); }
 };
 
 template <int LAYOUT, int NB>
 struct KqRaw<NVF_Q5_K, LAYOUT, NB> {
   static constexpr int kBlock = 176;
-  u32x4 hdr;
-  uint32_t q[NB / 4], h[NB / 4];
-  __device__ __forceinline__ void load(const uint8_t* blk, int quarter, int part) {
-    hdr = ld16(blk);
-    const uint8_t* p = blk + 48 + 32 * quarter + NB * part;
-    const uint8_t* ph = blk + 16 + NB * part;
-    if constexpr (NB == 16) {
-      const u32x4 v = ld16(p), g = ld16(ph);
+  struct Head {
+    u32x4 w;
+    uint32_t h[NB / 4];
+    __device__ __forceinline__ void load(const uint8_t* blk, int part) {
+      w = ld16(blk);
+      const uint8_t* p = blk + 16 + NB * part;
+      if constexpr (NB == 16) {
+        const u32x4 g = ld16(p);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        q[i] = v[i];
-        h[i] = g[i];
+        for (int i = 0; i < 4; ++i) h[i] = g[i];
+      } else {
+        const uint2 g = *reinterpret_cast<const uint2*>(p);
+        h[0] = g.x;
+        h[1] = g.y;
       }
+    }
+  } hd;
+  uint32_t q[NB / 4];
+  __device__ __forceinline__ void load(const uint8_t* blk, int quarter, int part) {
+    const uint8_t* p = blk + 48 + 32 * quarter + NB * part;
+    if constexpr (NB == 16) {
+      const u32x4 v = ld16(p);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q[i] = v[i];
     } else {
-      const uint2 v = *reinterpret_cast<const uint2*>(p), g = *reinterpret_cast<const uint2*>(ph);
+      const uint2 v = *reinterpret_cast<const uint2*>(p);
       q[0] = v.x;
       q[1] = v.y;
-      h[0] = g.x;
-      h[1] = g.y;
     }
   }
   static constexpr int kRuns = NB / 4;
@@ -107,13 +120,13 @@ struct KqRaw<NVF_Q5_K, LAYOUT, NB> {
     j = 2 * quarter + nib;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      b[i] = ((q[2 * u + i] >> (4 * nib)) & 0x0f0f0f0fu) | (((h[2 * u + i] >> j) & 0x01010101u) << 4);
+      b[i] = ((q[2 * u + i] >> (4 * nib)) & 0x0f0f0f0fu) | (((hd.h[2 * u + i] >> j) & 0x01010101u) << 4);
   }
   __device__ __forceinline__ void scale_min(int j, uint32_t& sc, uint32_t& mn) const {
-    q4k_sm(hdr[1], hdr[2], hdr[3], j, sc, mn);
+    q4k_sm(hd.w[1], hd.w[2], hd.w[3], j, sc, mn);
   }
-  __device__ __forceinline__ float d() const { return half_bits_to_f32(hdr[0] & 0xffffu); }
-  __device__ __forceinline__ float dmin() const { return half_bits_to_f32(hdr[0] >> 16); }
+  __device__ __forceinline__ float d() const { return half_bits_to_f32(hd.w[0] & 0xffffu); }
+  __device__ __forceinline__ float dmin() const { return half_bits_to_f32(hd.w[0] >> 16); }
 };
 
 template <int NB>
@@ -125,6 +138,9 @@ __device__ __forceinline__ void kq_load_a2(const uint8_t* p, uint32_t* out) {  /
 template <int LAYOUT, int NB>
 struct KqRaw<NVF_Q6_K, LAYOUT, NB> {  // element 128 h + 32 s + l: ql[64 h + 32 (s & 1) + l] nibble s / 2, qh[32 h + l]
   static constexpr int kBlock = 210;
+  struct Head {  // its header bytes differ between the stages
+    __device__ __forceinline__ void load(const uint8_t*, int) {}
+  } hd;
   uint32_t q[2][NB / 4], h[NB / 4];
   uint32_t sc[2];  // the int8 scales of slots s = 2 (quarter & 1), + 1 at this thread's l
   uint32_t dbits;
@@ -282,6 +298,7 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
     const int s = st < nst ? st : nst - 1;
     r.load(wrow + (int64_t)(s >> 2) * Raw::kBlock, s & 3, part);
   };
+  typename Raw::Head head, next;  // of the stage that is decoded, and of the superblock after it
   auto store_w = [&](const Raw& r, int st, int quarter, int buf) {
     uint8_t* base = lds + buf * L::kStage + L::kX + wc * kRowB;
 #pragma unroll
@@ -336,13 +353,13 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
 #pragma unroll
   for (int a = 0; a < TM; ++a)
 #pragma unroll
-    for (int b = 0; b < TN; ++b) acc[a][b] = blk[a][b] = f32x16{};
+    for (int b = 0; b < TN; ++b) acc[a][b] = f32x16{};
   const int half = lane >> 5, lr = lane & 31;
   const int ar = wm * TM * 32 + lr, br = wn * TN * 32 + lr;
   const int a0 = ar * kRowB + ((half ^ g16_key<64>(ar)) << 4);
   const int b0 = L::kX + br * kRowB + ((half ^ g16_key<64>(br)) << 4);
 
-  auto apply = [&](int sb) {  // acc += d B - dmin M, B = 0
+  auto apply = [&](int sb) {  // acc += d B - dmin M (the next superblock's first products start from 0)
     const int par = sb & 1;
 #pragma unroll
     for (int b = 0; b < TN; ++b) {
@@ -366,7 +383,6 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
           if constexpr (L::kMin) v = fmaf(-dd.y, t[j], v);
           acc[a][b][j] = v;
         }
-        blk[a][b] = f32x16{};
       }
     }
   };
@@ -374,6 +390,8 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
   issue(0, 0);
   load(raw[0], 0);
   load(raw[1], 1);
+  head.load(wrow, part);
+  next = raw[0].hd = head;
   store_w(raw[0], 0, 0, 0);
 #pragma unroll 1
   for (int sb = 0; sb < nsb; ++sb) {
@@ -388,6 +406,8 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
       if (q == 0 && sb > 0) apply(sb - 1);
       issue(st + 1, (q + 1) & 1);
       load(raw[q & 1], st + 2);
+      if (q == 2) next.load(wrow + (int64_t)(sb + 1 < nsb ? sb + 1 : sb) * Raw::kBlock, part);
+      __builtin_amdgcn_sched_barrier(0);  // the loads go out before the products, not after
       const uint8_t* s = lds + (q & 1) * L::kStage;
 #pragma unroll
       for (int kk = 0; kk < kKqBK / 16; ++kk) {
@@ -402,10 +422,13 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
 #pragma unroll
           for (int a = 0; a < TM; ++a)
 #pragma unroll
-            for (int b = 0; b < TN; ++b) blk[a][b] = mfma16(xa[a], wb[b], blk[a][b], T{});
+            for (int b = 0; b < TN; ++b)
+              blk[a][b] = mfma16(xa[a], wb[b], q == 0 && kk == 0 && p == L::kPlanes - 1 ? f32x16{} : blk[a][b], T{});
         }
       }
       sums(st, q & 1);
+      if (q == 3) head = next;
+      raw[(q + 1) & 1].hd = head;
       store_w(raw[(q + 1) & 1], st + 1, (q + 1) & 3, (q + 1) & 1);
     }
   }
