@@ -15,8 +15,9 @@
 //
 // 1021 x 37888 x 3584, fp16 x, Q4_K: the fp32 matrix-core tile kernel takes 2487 us (111
 // TFLOP/s), this one 406 (683; 430 with the
-// headers read in every stage, the loads left behind the products and B set to 0 by moves).  Activations reach LDS by DMA; a weight stage is loaded to registers two
-// stages ahead, decoded once per workgroup and stored to LDS as 16-bit operands.
+// headers read in every stage, the loads left behind the products and B set to 0 by moves).
+// Activations reach LDS by DMA; a weight stage is loaded to registers two stages ahead,
+// decoded once per workgroup and stored to LDS as 16-bit operands.
 //
 // Infinities and NaN: x and P are multiplied apart from the weight's scale and offset, so a
 // non-finite activation or superblock scale (or an activation beyond 1e35) can give NaN
