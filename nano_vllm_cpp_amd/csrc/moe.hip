@@ -640,9 +640,11 @@ __global__ __launch_bounds__(WM* WN* KG * 64) __attribute__((amdgpu_waves_per_eu
 
     // the tile in LDS as fp32 [BM][BN], the K groups adding their sums in group order
     constexpr int kPitch = BN * 4 + 16;
+    uint32_t* const bad_at = reinterpret_cast<uint32_t*>(lds + BM * kPitch);  // [wave]: a non-finite sum
 #pragma unroll 1
     for (int g = 0; g < KG; ++g) {
       if (group == g) {
+        bool bad = false;
 #pragma unroll
         for (int b = 0; b < TM; ++b)
 #pragma unroll
@@ -660,9 +662,72 @@ __global__ __launch_bounds__(WM* WN* KG * 64) __attribute__((amdgpu_waves_per_eu
                 for (int e = 0; e < 4; ++e) v[e] += o[e];
               }
               st16(d, Pack<float>::pack(v));
+              if constexpr (XP > 1) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bad = bad || !__builtin_isfinite(v[e]);
+              }
             }
+        if constexpr (XP > 1) {
+          const uint64_t any = __ballot(bad);
+          if (g == KG - 1 && lane == 0) bad_at[wave] = any != 0;
+        }
       }
       __syncthreads();
+    }
+
+    // A plane of zeros times an infinite weight is NaN, where the value itself times that
+    // weight is an infinity: non-finite sums are made again on the fp32 matrix cores from the
+    // whole values (the planes' exact sums), 32 x 32 results of the tile per wave and turn.
+    if constexpr (XP > 1) {
+      uint32_t any = 0;
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) any |= bad_at[i];
+      if (any) {  // the same in every wave
+#pragma unroll 1
+        for (int u = wave_id; u < (BM / 32) * (BN / 32); u += kWaves * KG) {
+          const int b = u / (BN / 32), a = u % (BN / 32), col = 32 * a + lr;
+          const int64_t pos = t.pos0 + 32 * b + lr;
+          const bool x_ok = pos < t.pos_end;
+          uint8_t* const d = lds + (32 * b + lr) * kPitch + (32 * a + 4 * half) * 4;
+          float o[16];
+          bool bad = false;
+#pragma unroll
+          for (int jq = 0; jq < 4; ++jq) Pack<float>::unpack(ld16(d + 32 * jq), o + 4 * jq);
+#pragma unroll
+          for (int j = 0; j < 16; ++j) bad = bad || !__builtin_isfinite(o[j]);
+          if (!__any(bad && x_ok)) continue;
+          const int64_t cc = t.col0 + (GU ? col % (BN / 2) : col);
+          const bool w_ok = cc < prob.n_cols;
+          const __bf16* xrow = xp + (x_ok ? (GU ? (int64_t)prob.list[pos] / x_per : pos) : 0) * k;
+          const __bf16* wrow = wbase + (w_ok ? (GU && col >= BN / 2 ? prob.n_cols + cc : cc) : 0) * k;
+          f32x16 v = f32x16{};
+#pragma unroll 1
+          for (int64_t e = 0; e < k; e += 16) {
+            const int64_t e8 = e + 8 * half;
+            float wv[8] = {}, xv[8] = {};
+            if (e8 < k && w_ok) Pack<__bf16>::unpack(ld16(wrow + e8), wv);
+            if (e8 < k && x_ok) {
+#pragma unroll
+              for (int p = 0; p < XP; ++p) {
+                float pv[8];
+                Pack<__bf16>::unpack(ld16(xrow + p * plane + e8), pv);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) xv[i] += pv[i];
+              }
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[i], xv[i], v, 0, 0, 0);
+          }
+#pragma unroll
+          for (int jq = 0; jq < 4; ++jq) {
+            float r[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[e] = __builtin_isfinite(o[4 * jq + e]) ? o[4 * jq + e] : v[4 * jq + e];
+            st16(d + 32 * jq, Pack<float>::pack(r));
+          }
+        }
+        __syncthreads();
+      }
     }
     constexpr int kThreads = kWaves * KG * 64;
     if constexpr (GU) {
@@ -771,7 +836,7 @@ int moe_product(const TX* a, const TW* w, Prob prob, int64_t k, const MoePlan& p
 template <bool GU, int XP, int BM, int BN, int WM, int WN, int KG, int NS, int OCC>
 int launch_moe16(const __bf16* xp, int64_t plane, int64_t x_per, const __bf16* w, MoeTiles prob, int64_t k, __bf16* yp,
                  int64_t yplane, float* v, int64_t max_tiles, hipStream_t st) {
-  constexpr int kRing = KG * NS * (XP * BM + BN) * 128, kEpi = BM * (BN * 4 + 16), kLds = kRing > kEpi ? kRing : kEpi;
+  constexpr int kRing = KG * NS * (XP * BM + BN) * 128, kEpi = BM * (BN * 4 + 16) + WM * WN * 4, kLds = kRing > kEpi ? kRing : kEpi;
   auto kern = moe16_kernel<GU, XP, BM, BN, WM, WN, KG, NS, OCC>;
   static std::once_flag attr_once;
   std::call_once(attr_once, [&] {

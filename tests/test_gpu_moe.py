@@ -268,3 +268,44 @@ def test_moe_ffn_bf16_tiles(gpu, x_dt, rows, hid, inter, k, n_exp, slots):
     got = ops.moe_ffn(H.to_dev(x, gpu, x_dt), H.to_dev(idx, gpu), H.to_dev(score, gpu), H.to_dev(gu, gpu, H.BF16),
                       H.to_dev(dn, gpu, H.BF16), H.to_dev(slot_of, gpu), inter, slots, H.to_dev(out_in, gpu, H.F32))
     assert_within(H.to_host(got), ideal, err, H.F32, "moe_ffn bf16 tiles", True)
+
+
+@pytest.mark.parametrize("x_dt", DTYPES, ids=DT_IDS)
+@pytest.mark.parametrize("rows,k", [(7, 2), (24, 2), (530, 8), (2050, 8)],
+                         ids=["64 columns", "32 rows", "64 rows", "128 rows"])
+def test_moe_ffn_bf16_infinities(gpu, x_dt, rows, k):
+    """Infinite activations, gate, up and down weights on every tile shape: infinities and NaN
+    where the plain products of the same operands put them."""
+    if rows == 7 and x_dt != H.BF16:
+        pytest.skip("fewer than 16 pairs with fp16 or fp32 x take the decode product, not these tiles")
+    r = H.rng(rows + x_dt)
+    hid, inter, n_exp = 136, 40, 12 * k
+    x, gu, dn, idx, score, slot_of = moe_case(r, rows, hid, inter, k, n_exp, n_exp, True, x_dt)
+    for t in range(5):  # rows 0 to 4 meet the slots with infinite weights
+        e = int(np.flatnonzero(slot_of == t)[0])
+        if e not in idx[t]:
+            idx[t, 0] = e
+    inf = 0x7F80
+    x[3, 7] = {H.F32: np.inf, H.F16: 0x7C00, H.BF16: inf}[x_dt]
+    x[:, 50] = H.to_storage(np.full(rows, 1.25, np.float32), x_dt)  # one bf16 piece: the others are 0
+    gu[0, 5, 50], gu[1, inter + 9, 50] = inf, inf                     # a gate row, an up row
+    gu[2, 6, 51] = inf                                                # pieces of either sign
+    dn[3, 11, 20], dn[4, 12, 20] = inf, inf | 0x8000
+    f = [H.from_storage(a, dt).astype(np.float64) for a, dt in ((x, x_dt), (gu, H.BF16), (dn, H.BF16))]
+    want = np.zeros((rows, hid))
+    with np.errstate(all="ignore"):
+        for t in range(rows):
+            for j in range(k):
+                s = slot_of[idx[t, j]]
+                g = (f[1][s] * f[0][t]).sum(-1)
+                y = g[:inter] / (1.0 + np.exp(-g[:inter])) * g[inter:]
+                want[t] += np.float64(score[t, j]) * (f[2][s] * y).sum(-1)
+    assert np.isinf(want).any() and np.isnan(want).any() and np.isfinite(want).any()
+    case(f"nvf_moe_ffn infinities x={x_dt} rows={rows} K={k}")
+    got = H.to_host(ops.moe_ffn(H.to_dev(x, gpu, x_dt), H.to_dev(idx, gpu), H.to_dev(score, gpu),
+                                H.to_dev(gu, gpu, H.BF16), H.to_dev(dn, gpu, H.BF16), H.to_dev(slot_of, gpu), inter,
+                                n_exp, torch.zeros(rows, hid, device=gpu)))
+    for what, is_it in (("NaN", np.isnan), ("+inf", np.isposinf), ("-inf", np.isneginf)):
+        np.testing.assert_array_equal(is_it(got), is_it(want), what)
+    fin = np.isfinite(want)
+    assert np.allclose(got[fin], want[fin], rtol=1e-4, atol=1e-4 * np.abs(want[fin]).max())
