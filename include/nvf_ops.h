@@ -235,8 +235,11 @@ int nvf_add_bias(void* x, const float* bias, int64_t rows, int64_t cols, int64_t
 
 /* GEMM on dense or K-quant weights (replaces hip_matmul, hip_matmul_u16 and
  * hip_matmul_qk, hip_ops.hpp:8-11): out[m,n] (out_dtype) = x[m,k] (x_dtype) . w^T with
- * w in `w_format` (nvf_w_format; Q4_K nibble order `qk_layout`) decoded exactly to fp32,
- * fp32 products and sums on the matrix cores.  Any k; K-quants: n*k a multiple of 256,
+ * w in `w_format` (nvf_w_format; Q4_K nibble order `qk_layout`), exact products, fp32 sums:
+ * within c (k + 2) 2^-24 sum |x w| of the exact result (before out_dtype's rounding), c = 1;
+ * fp16 / bf16 weights on the split products 6 / 3; K-quants that go to the 16-bit matrix
+ * cores 3 (each weight as two parts, d sc (q - c) and the rest, of at most three times its size).
+ * Any k; K-quants: n*k a multiple of 256,
  * Q4_K/Q5_K blocks 16-byte aligned, Q6_K 2-byte.  Vector loads when x and dense
  * weights are 16-byte aligned, element-wise staging otherwise. */
 int nvf_matmul(const void* x, int x_dtype, const void* w, int w_format, int qk_layout, int64_t m, int64_t n,

@@ -1,5 +1,5 @@
 // GEMM on fp32 / fp16 / bf16 and K-quant (Q4_K, Q5_K, Q6_K) weights: out[r][c] = sum_i
-// x[r][i] * w(c, i), the weights decoded exactly.
+// x[r][i] * w(c, i), the weights' values exact.
 //
 // Reference: hip_matmul (matmul_kernel<float>, src/hip_ops.hip:43-64), hip_matmul_u16
 // (matmul_kernel<uint16_t>: fp16/bf16 weights widened exactly) and hip_matmul_qk
@@ -12,9 +12,12 @@
 // Design for gfx950: activations and weights of one 16-bit type go to the 16-bit matrix
 // cores as they are (gemm16.hpp, m > 2); otherwise the tile kernels of gemm_tile.hpp
 // for m > 16 (m <= 32 takes 32-row tiles, so a small m does not multiply the
-// matrix-core work), and the weight-streaming decode products below for m <= 16.  The sums are fp32
-// in a different order from the reference's, so results agree within the
-// recursive-summation bound the tests state.
+// matrix-core work), and the weight-streaming decode products below for m <= 16.  K-quants go
+// to kq_gemm.hip (16-bit x, m > 16) and kq_gemv.hip (Q4_K / Q5_K, m <= 16 where it wins).
+// The sums are fp32 in a different order from the reference's, so results agree within the
+// recursive-summation bound (k + 2) 2^-24 sum |x w| that the tests state; the two K-quant
+// kernels sum a weight's two parts apart, at most three times as large as the weight together,
+// so theirs is three times that.
 
 #include "nvf_device.hpp"
 #include "nvf_host.hpp"
@@ -339,20 +342,26 @@ int launch_dense(const void* x, const Src& src, void* out, int64_t m, int64_t n,
 // Where the 16-bit matrix-core decode product of kq_gemv.hip beats the products on decoded
 // weights above.  Q4_K, us (there / here), weights not in the cache:
 //   fp16 x, m =                1            2            4            8            16
-//   151936 x 4096        67 / 136     75 / 155     79 / 247     94 / 249    124 / 254
-//   37888 x 3584       22.5 / 29.5  21.5 / 36.1  23.1 / 58.9  27.2 / 59.2  35.9 / 61.4
-//   4608 x 3584         7.7 / 6.9    8.8 / 8.4   10.2 / 14.3  13.2 / 14.5  19.6 / 15.2
-//   3584 x 18944       14.3 / 17.1  17.3 / 21.6  22.5 / 38.3  32.4 / 38.8  52.1 / 39.2
+//   151936 x 4096        82 / 136     80 / 153     86 / 247    101 / 249    130 / 253
+//   37888 x 3584       22.8 / 26.4  24.3 / 33.4  25.2 / 55.0  29.2 / 56.1  37.8 / 58.1
+//   4608 x 3584             / 9.9        / 9.8   12.0 / 14.6  15.7 / 14.7       / 15.5
+//   3584 x 18944       17.4 / 17.1  19.6 / 22.9  25.0 / 38.6  35.1 / 38.8       / 38.8
+//   bf16 x
+//   151936 x 4096        91 / 132     95 / 153    101 / 246    117 / 248    147 / 252
+//   37888 x 3584       29.8 / 27.2  30.4 / 38.9  31.4 / 54.5  35.5 / 55.2  43.5 / 56.8
+//   4608 x 3584             / 9.9        / 9.8   13.1 / 14.1  16.4 / 14.3       / 15.3
+//   3584 x 18944            / 17.2  23.3 / 23.1  27.8 / 38.3  37.9 / 38.3       / 38.5
 //   fp32 x
-//   37888 x 3584       33.3 / 33.1  34.2 / 45.6  37.4 / 54.9  43.8 / 57.3  69.3 / 69.3
-//   4608 x 3584        12.2 / 8.1   12.3 / 11.8  14.9 / 14.1  26.8 / 14.8  41.5 / 19.2
-//   3584 x 18944       25.2 / 20.4  25.7 / 31.4  32.4 / 35.1  68.1 / 36.0
-// (bf16 x: as fp16, a little slower; 1 x 3584 x 18944 18.4 / 17.1).  Narrow outputs have few
-// workgroups over which to spread its staging of x.
-bool kq_gemv_wins(int x_dtype, int64_t m, int64_t n, int64_t k) {
-  if (n >= 16384) return true;
-  if (x_dtype == NVF_F32) return m >= 2 && m <= 4 && k >= 8192;
-  return m <= 8 && (m > 2 || (k >= 8192 && (m == 2 || x_dtype == NVF_F16)));
+//   151936 x 4096       112 / 153    115 / 194    126 / 247    150 / 252    227 / 266
+//   37888 x 3584       34.4 / 32.0  34.7 / 45.5  37.9 / 54.5  44.7 / 57.0  70.8 / 70.3
+//   3584 x 18944            / 22.5  27.3 / 33.8  34.3 / 35.4       / 35.4       / 44.0
+// (Q5_K, one row, 37888 x 3584: fp16 29.1 / 39.4, bf16 34.9 / 39.2, fp32 39.4 / 46.1.)  Narrow
+// outputs have few workgroups over which to spread its staging of x.
+bool kq_gemv_wins(int w_format, int x_dtype, int64_t m, int64_t n, int64_t k) {
+  const bool f16 = x_dtype == NVF_F16, deep = k >= 8192;
+  if (n >= 16384) return m > 1 || f16 || w_format == NVF_W_Q5_K || n >= 65536;
+  if (x_dtype == NVF_F32) return m >= 2 && m <= 4 && deep;
+  return m >= (f16 && deep ? 2 : 3) && m <= (deep ? 8 : 4);
 }
 
 template <typename TX, typename TO>
@@ -360,7 +369,7 @@ int dispatch_weights(const void* x, const void* w, int w_format, int layout, voi
                      int64_t k, bool vec, hipStream_t st) {
   const uint8_t* wb = static_cast<const uint8_t*>(w);
   if ((w_format == NVF_W_Q4_K || w_format == NVF_W_Q5_K) && vec && m <= kGemvRows && k % 256 == 0 &&
-      k < (1 << 22) && kq_gemv_wins(dtype_of<TX>(), m, n, k))
+      k < (1 << 22) && kq_gemv_wins(w_format, dtype_of<TX>(), m, n, k))
     return kq_gemv(x, dtype_of<TX>(), w, w_format, layout, out, dtype_of<TO>(), m, n, k, st);
   if constexpr (sizeof(TX) == 2) {  // whole superblocks per row: the 16-bit matrix cores
     if (w_format >= NVF_W_Q4_K && vec && m > kGemvRows && k % 256 == 0 && k < (1 << 22))

@@ -2,20 +2,23 @@
 // matrix cores: out[m][n] = x[m][k] . W[n][k]^T, k a multiple of 256 (whole superblocks
 // per weight row), m > 16.
 //
-// A weight of a superblock is d sc_j q - dmin m_j (Q6_K: d sc_j (q - 32)) with 6-bit
-// (Q6_K: signed 8-bit) whole sc_j, m_j of its sub-block and a whole q.  The integer
-// P = sc_j q has at most 11 significant bits (Q6_K 13), so it is one fp16 value exactly, or
-// the exact sum of two 16-bit values.  Per superblock the matrix cores sum
+// A weight of a superblock is d sc_j q - dmin m_j with 6-bit whole sc_j, m_j of its sub-block and
+// a whole q.  With the sub-block's centre c_j (kq_centre: the quant nearest to where the weight
+// is 0) it is d sc_j (q - c_j) + r_j, r_j = d sc_j c_j - dmin m_j in fp32; Q6_K is d sc_j (q - 32),
+// sc_j signed 8-bit.  The integer P = sc_j (q - c_j) has at most 11 significant bits (Q6_K 13), so
+// it is one fp16 value exactly, or the exact sum of two 16-bit values.  Per superblock the matrix
+// cores sum
 //   B = sum_k x_k P_k                (exact products, fp32 sums)
-//   M = sum_j m_j (sum_{k in j} x_k) (Q4_K / Q5_K: the sub-block sums of x as three exact
-//                                    bf16 pieces, so these products are exact too)
-// and the accumulator takes d B - dmin M: two fused multiply-adds per output and 256 K,
-// where a scale per sub-block would cost them per 32 K and decoding each weight to fp32
-// leaves only the fp32 matrix cores, 16 times slower.
+//   R = sum_j r_j (sum_{k in j} x_k) (the sub-block sums of x and the r_j as three bf16 pieces
+//                                    each, the six products down to 2^-24 of the largest)
+// and the accumulator takes R, and d B by one fused multiply-add per output and 256 K, where a
+// scale per sub-block would cost one per 32 K and decoding each weight to fp32
+// leaves only the fp32 matrix cores, 16 times slower.  P and r_j are at most twice and once
+// their weight, so the result is within three times the bound of fp32 sums of x w.
 //
 // 1021 x 37888 x 3584, fp16 x, Q4_K: the fp32 matrix-core tile kernel takes 2487 us (111
-// TFLOP/s), this one 406 (683; 430 with the
-// headers read in every stage, the loads left behind the products and B set to 0 by moves).
+// TFLOP/s), this one 407 (681; 399 with c_j = 0, whose two parts can cancel: then the error is
+// bounded by sums of |x| (d sc q + dmin m) alone; 421 with the centres found behind the products).
 // Activations reach LDS by DMA; a weight stage is loaded to registers two stages ahead,
 // decoded once per workgroup and stored to LDS as 16-bit operands.
 //
@@ -26,6 +29,7 @@
 
 #include <array>
 #include <mutex>
+#include <type_traits>
 
 #include "gemm16.hpp"
 #include "gemm_tile.hpp"
@@ -36,7 +40,8 @@ constexpr int kKqBN = 128, kKqBK = 64;
 
 // One stage of one thread: NB bytes of quants of column c, part p of its 64 K values.  Head is
 // what a superblock's four stages share, loaded once for them: read again in every
-// stage, the compiler merges it with the older copy and waits for the newest load.  put() hands (chunk, 8 integers q as bytes, scale index) on.
+// stage, the compiler merges it with the older copy and waits for the newest load.  run() gives (8 integers q as
+// bytes, chunk, scale index).
 template <int KIND, int LAYOUT, int NB>
 struct KqRaw;
 
@@ -172,44 +177,46 @@ struct KqRaw<NVF_Q6_K, LAYOUT, NB> {  // element 128 h + 32 s + l: ql[64 h + 32 
   __device__ __forceinline__ float dmin() const { return 0.0f; }
 };
 
-// 16-bit operand planes of 8 integers P = sc q (Q6_K: sc (q - 32), sc signed), the q as
-// bytes: the planes sum to P exactly.
+// 16-bit operand planes of 8 integers P = sc (q - q0) (Q6_K: sc (q - 32), sc signed), the q as
+// bytes and q0 the sub-block's centre: the planes sum to P exactly.
 template <typename T, int KIND>
 struct KqPlanes {
   static constexpr int value = __is_same(T, _Float16) && KIND != NVF_Q6_K ? 1 : 2;
 };
+// 1 / the planes' unit.
+template <typename T, int KIND>
+constexpr float kKqUnit = __is_same(T, _Float16) && KIND != NVF_Q6_K ? 0x1p14f : 1.0f;
 template <int KIND>
-__device__ __forceinline__ void kq_planes(const uint32_t* b, uint32_t sc, u32x4* p, _Float16) {
-  // bytes under 0x64: the fp16 value 1024 + q
-  const uint32_t magic = 0x64646464u;
+__device__ __forceinline__ void kq_planes(const uint32_t* b, uint32_t sc, uint32_t q0, u32x4* p, _Float16) {
+  // Q4_K, Q5_K: a byte under a zero one is the subnormal q 2^-24, and one exact multiply-add
+  // makes it sc (q - q0) 2^-14.  Q6_K: bytes under 0x64 are the fp16 values 1024 + q.
+  const uint32_t top = KIND == NVF_Q6_K ? 0x64646464u : 0u;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t w = b[i >> 1];
-    const f16x2 t = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(magic, w, (i & 1) ? 0x07030602u : 0x05010400u));
+    const f16x2 t = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(top, w, (i & 1) ? 0x07030602u : 0x05010400u));
     if constexpr (KIND == NVF_Q6_K) {
       const int s = (int8_t)sc, lo = s & 15, hi = s - lo;  // s = hi + lo, hi a multiple of 16
       const f16x2 q = t - f16x2{(_Float16)1056.0f, (_Float16)1056.0f};
       const f16x2 l2 = {(_Float16)(float)lo, (_Float16)(float)lo}, h2 = {(_Float16)(float)hi, (_Float16)(float)hi};
       p[0][i] = __builtin_bit_cast(uint32_t, q * h2);
       p[1][i] = __builtin_bit_cast(uint32_t, q * l2);
-    } else {  // (1024 + q) sc - 1024 sc, one rounding of an exact value (1024 sc <= 64512)
-      const _Float16 s = (_Float16)(float)sc, c = (_Float16)(-1024.0f * (float)sc);
+    } else {
+      const _Float16 s = (_Float16)(1024.0f * (float)sc), c = (_Float16)(-0x1p-14f * (float)sc * (float)q0);
       const f16x2 s2 = {s, s}, c2 = {c, c};
       p[0][i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(t, s2, c2));
     }
   }
 }
 template <int KIND>
-__device__ __forceinline__ void kq_planes(const uint32_t* b, uint32_t sc, u32x4* p, __bf16) {
-  const float s = KIND == NVF_Q6_K ? (float)(int8_t)sc : (float)sc;
+__device__ __forceinline__ void kq_planes(const uint32_t* b, uint32_t sc, uint32_t q0, u32x4* p, __bf16) {
+  const float s = KIND == NVF_Q6_K ? (float)(int8_t)sc : (float)sc, c = s * (KIND == NVF_Q6_K ? -32.0f : -(float)q0);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     uint32_t hi[2], lo[2];
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      float q = (float)byte_of(b[i >> 1], 2 * (i & 1) + e);
-      if constexpr (KIND == NVF_Q6_K) q -= 32.0f;
-      const float v = q * s;  // a whole number below 2^13
+      const float v = fmaf((float)byte_of(b[i >> 1], 2 * (i & 1) + e), s, c);  // a whole number below 2^13
       hi[e] = __builtin_bit_cast(uint32_t, v) & 0xffff0000u;
       lo[e] = __builtin_bit_cast(uint32_t, v - __builtin_bit_cast(float, hi[e]));  // at most 8 bits: exact in bf16
     }
@@ -239,16 +246,16 @@ __device__ __forceinline__ float kq_sum8(u32x4 v, float s, __bf16) {
 }
 
 template <typename T, int KIND, int BM, int WM, int WN>
-struct KqLds {  // byte offsets; two stage buffers, two of each table (superblock parity)
+struct KqLds {  // byte offsets; two stage buffers, two tables of x's sums (superblock parity)
   static constexpr int kPlanes = KqPlanes<T, KIND>::value;
   static constexpr int kX = BM * kKqBK * 2, kW = kKqBN * kKqBK * 2;
   static constexpr int kStage = kX + kPlanes * kW;
   static constexpr bool kMin = KIND != NVF_Q6_K;
-  static constexpr int kXs = kMin ? BM * 48 : 0;      // x sub-block sums: [piece][row][8 j] bf16
-  static constexpr int kMn = kMin ? kKqBN * 16 : 0;   // m_j: [column][8 j] bf16
-  static constexpr int kD = kKqBN * 8;                // d, dmin
-  static constexpr int kXsAt = 2 * kStage, kMnAt = kXsAt + 2 * kXs, kDAt = kMnAt + 2 * kMn;
-  static constexpr int kBytes = kDAt + 2 * kD;
+  static constexpr int kXs = kMin ? BM * 48 : 0;     // x sub-block sums: [piece][row][8 j] bf16
+  static constexpr int kR = kMin ? kKqBN * 48 : 0;   // r_j: [piece][column][8 j] bf16
+  static constexpr int kD = kKqBN * 4;               // d
+  static constexpr int kXsAt = 2 * kStage, kRAt = kXsAt + 2 * kXs, kDAt = kRAt + kR;
+  static constexpr int kBytes = kDAt + (kMin ? kD : 2 * kD);
 };
 
 template <typename T, int KIND, int LAYOUT, typename TO, int BM, int WM, int WN>
@@ -300,6 +307,45 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
     r.load(wrow + (int64_t)(s >> 2) * Raw::kBlock, s & 3, part);
   };
   typename Raw::Head head, next;  // of the stage that is decoded, and of the superblock after it
+  uint32_t cen[2] = {};           // its centres c_j, one per byte
+  uint32_t rem[4 / kTpc][3] = {};  // the r_j that this thread finds, in pairs: three pieces
+  // the column's threads find 8 / kTpc centres each and hand them round (quad_perm)
+  auto centres = [&](const Raw& r) {
+    if constexpr (L::kMin) {
+      constexpr int kOwn = 8 / kTpc;
+      uint32_t sc[2], mn[2];
+      q4k_tables(r.hd.w, sc, mn);
+      const int sh = kTpc == 2 ? 0 : 16 * (part & 1);
+      const bool low = part < kTpc / 2;  // this thread's are among c_0 .. c_3
+      const uint32_t sw = (low ? sc[0] : sc[1]) >> sh, mw = (low ? mn[0] : mn[1]) >> sh;
+      const float d = r.d(), dmin = r.dmin();
+      uint32_t own = 0, pc[kOwn][3];
+#pragma unroll
+      for (int i = 0; i < kOwn; ++i) {
+        const float p = d * (float)byte_of(sw, i), o = dmin * (float)byte_of(mw, i);
+        const float c = kq_centre(p, o, KIND == NVF_Q4_K ? 15.0f : 31.0f);
+        own |= (uint32_t)c << (8 * i);
+        bf16_pieces(fmaf(p, c, -o), pc[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < kOwn / 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) rem[i][q] = pc[2 * i][q] | pc[2 * i + 1][q] << 16;
+      auto swap = [](uint32_t v, auto ctrl) {
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xf, 0xf, false);
+      };
+      uint32_t other;
+      if constexpr (kTpc == 2) {
+        other = swap(own, std::integral_constant<int, 0xb1>{});
+      } else {
+        own <<= sh;
+        own |= swap(own, std::integral_constant<int, 0xb1>{});
+        other = swap(own, std::integral_constant<int, 0x4e>{});
+      }
+      cen[0] = low ? own : other;
+      cen[1] = low ? other : own;
+    }
+  };
   auto store_w = [&](const Raw& r, int st, int quarter, int buf) {
     uint8_t* base = lds + buf * L::kStage + L::kX + wc * kRowB;
 #pragma unroll
@@ -309,25 +355,24 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
       r.run(u, quarter, part, b, chunk, j);
       r.scale_min(j, sc, mn);
       u32x4 p[2];
-      kq_planes<KIND>(b, sc, p, T{});
+      kq_planes<KIND>(b, sc, byte_of(cen[j >> 2], j & 3), p, T{});
 #pragma unroll
       for (int i = 0; i < L::kPlanes; ++i) st16(base + i * L::kW + ((chunk ^ wkey) << 4), p[i]);
     }
-    if (quarter == 0) {  // the superblock's d, dmin and m_j
-      const int par = (st >> 2) & 1;
+    // the superblock's d and r_j: after quarter 0, in which the last superblock's are still read
+    if (quarter == 2) {
       if constexpr (L::kMin) {
 #pragma unroll
-        for (int i = 0; i < 4 / kTpc; ++i) {
-          uint32_t sc, m0, m1;
-          const int jp = part * (4 / kTpc) + i;
-          r.scale_min(2 * jp, sc, m0);
-          r.scale_min(2 * jp + 1, sc, m1);
-          const uint32_t f0 = __builtin_bit_cast(uint32_t, (float)m0), f1 = __builtin_bit_cast(uint32_t, (float)m1);
-          *reinterpret_cast<uint32_t*>(lds + L::kMnAt + par * L::kMn + wc * 16 + jp * 4) = (f0 >> 16) | f1;
-        }
+        for (int i = 0; i < 4 / kTpc; ++i)
+#pragma unroll
+          for (int q = 0; q < 3; ++q)
+            *reinterpret_cast<uint32_t*>(lds + L::kRAt + q * (kKqBN * 16) + wc * 16 + (part * (4 / kTpc) + i) * 4) =
+                rem[i][q];
       }
-      if (part == 0) *reinterpret_cast<float2*>(lds + L::kDAt + par * L::kD + wc * 8) = make_float2(r.d(), r.dmin());
+      if (L::kMin && part == 0) *reinterpret_cast<float*>(lds + L::kDAt + wc * 4) = r.d() * kKqUnit<T, KIND>;
     }
+    if (!L::kMin && quarter == 0 && part == 0)
+      *reinterpret_cast<float*>(lds + L::kDAt + ((st >> 2) & 1) * (kKqBN * 4) + wc * 4) = r.d();
   };
 
   // sub-block sums of the stage's activations, as three bf16 pieces
@@ -340,13 +385,11 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
       float v = 0.0f;
 #pragma unroll
       for (int c = 0; c < 4; ++c) v = kq_sum8(ld16(p + (((4 * s + c) ^ key) << 4)), v, T{});
-      const uint32_t h = __builtin_bit_cast(uint32_t, v) & 0xffff0000u;
-      const float r1 = v - __builtin_bit_cast(float, h);
-      const __bf16 b1 = (__bf16)r1, b2 = (__bf16)(r1 - (float)b1);
+      uint32_t pc[3];
+      bf16_pieces(v, pc);
       uint16_t* d = reinterpret_cast<uint16_t*>(lds + L::kXsAt + par * L::kXs) + r * 8 + 2 * quarter + s;
-      d[0] = (uint16_t)(h >> 16);
-      d[BM * 8] = __builtin_bit_cast(uint16_t, b1);
-      d[2 * BM * 8] = __builtin_bit_cast(uint16_t, b2);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) d[q * BM * 8] = (uint16_t)pc[q];
     }
   };
 
@@ -360,30 +403,29 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
   const int a0 = ar * kRowB + ((half ^ g16_key<64>(ar)) << 4);
   const int b0 = L::kX + br * kRowB + ((half ^ g16_key<64>(br)) << 4);
 
-  auto apply = [&](int sb) {  // acc += d B - dmin M (the next superblock's first products start from 0)
+  auto apply = [&](int sb) {  // acc += R + d B (the next superblock's first products start from 0)
     const int par = sb & 1;
 #pragma unroll
     for (int b = 0; b < TN; ++b) {
-      const float2 dd = *reinterpret_cast<const float2*>(lds + L::kDAt + par * L::kD + (br + 32 * b) * 8);
-      u32x4 mn = {};
-      if constexpr (L::kMin) mn = ld16(lds + L::kMnAt + par * L::kMn + (br + 32 * b) * 16);
+      const float d = *reinterpret_cast<const float*>(lds + L::kDAt + (L::kMin ? 0 : par * L::kD) + (br + 32 * b) * 4);
+      u32x4 r0 = {}, r1 = {}, r02 = {};
+      if constexpr (L::kMin) {  // k slots 0-7 (half 0) and 8-15 (half 1) of an MFMA
+        const uint8_t* rt = lds + L::kRAt + (br + 32 * b) * 16;
+        r0 = ld16(rt);
+        r1 = ld16(rt + kKqBN * 16);
+        r02 = ld16(rt + half * (2 * kKqBN * 16));
+      }
 #pragma unroll
       for (int a = 0; a < TM; ++a) {
-        f32x16 t = f32x16{};
         if constexpr (L::kMin) {
           const uint8_t* xs = lds + L::kXsAt + par * L::kXs + (ar + 32 * a) * 16;
-          const u32x4 x01 = ld16(xs + half * BM * 16);  // k slots 0-7: piece 0, 8-15: piece 1
-          u32x4 x2 = ld16(xs + 2 * BM * 16);            // k slots 0-7: piece 2
-          if (half) x2 = u32x4{};
-          t = mfma16(x2, mn, t, __bf16{});
-          t = mfma16(x01, mn, t, __bf16{});
+          const u32x4 x01 = ld16(xs + half * (BM * 16)), x20 = ld16(xs + (1 - half) * (2 * BM * 16));
+          acc[a][b] = mfma16(x20, r02, acc[a][b], __bf16{});
+          acc[a][b] = mfma16(x01, r1, acc[a][b], __bf16{});
+          acc[a][b] = mfma16(x01, r0, acc[a][b], __bf16{});
         }
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          float v = fmaf(dd.x, blk[a][b][j], acc[a][b][j]);
-          if constexpr (L::kMin) v = fmaf(-dd.y, t[j], v);
-          acc[a][b][j] = v;
-        }
+        for (int j = 0; j < 16; ++j) acc[a][b][j] = fmaf(d, blk[a][b][j], acc[a][b][j]);
       }
     }
   };
@@ -393,6 +435,7 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
   load(raw[1], 1);
   head.load(wrow, part);
   next = raw[0].hd = head;
+  centres(raw[0]);
   store_w(raw[0], 0, 0, 0);
 #pragma unroll 1
   for (int sb = 0; sb < nsb; ++sb) {
@@ -409,6 +452,9 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
       load(raw[q & 1], st + 2);
       if (q == 2) next.load(wrow + (int64_t)(sb + 1 < nsb ? sb + 1 : sb) * Raw::kBlock, part);
       __builtin_amdgcn_sched_barrier(0);  // the loads go out before the products, not after
+      if (q == 3) head = next;
+      raw[(q + 1) & 1].hd = head;
+      if (q == 3) centres(raw[(q + 1) & 1]);
       const uint8_t* s = lds + (q & 1) * L::kStage;
 #pragma unroll
       for (int kk = 0; kk < kKqBK / 16; ++kk) {
@@ -428,8 +474,6 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
         }
       }
       sums(st, q & 1);
-      if (q == 3) head = next;
-      raw[(q + 1) & 1].hd = head;
       store_w(raw[(q + 1) & 1], st + 1, (q + 1) & 3, (q + 1) & 1);
     }
   }

@@ -3,13 +3,14 @@
 //
 // Bound by the weights' stream from HBM as long as decoding them costs about 2 VALU
 // instructions per weight; decoding each to fp32 and multiplying on the VALU takes 5.2 at one
-// row, and the fp32 matrix cores are slower still.  Here only the whole quant q becomes a
-// 16-bit operand (for fp16 a mask: a subnormal; for bf16 a conversion), one
-// v_mfma_f32_16x16x32 sums a sub-block's 32 exact products x q for 16 rows and 16 columns, and
-// the sub-block's scale takes one fused multiply-add per four rows and 512 weights.  The
-// minimum's part is one MFMA per superblock, over the sub-blocks' sums of x (three exact bf16
-// pieces) and the m_j.  fp16 x takes fp16 operands; bf16 x bf16; fp32 x three exact
-// bf16 pieces.
+// row, and the fp32 matrix cores are slower still.  Here c_j is a sub-block's centre
+// (kq_centre) and r_j = d sc_j c_j - dmin m_j its remainder, as in kq_gemm.hip.  fp16 x: a weight's
+// quant is masked out as a subnormal and one packed multiply-add makes it the exact operand
+// sc_j (q - c_j) 2^-14, so v_mfma_f32_16x16x32 sums whole superblocks for 16 rows and 16 columns,
+// and d takes one fused multiply-add per four rows and 4096 weights.  bf16 x (and fp32 x as
+// three exact bf16 pieces): the operand is q - c_j, and sc_j takes one multiply-add per four rows
+// and 512 weights.  The r_j are two MFMAs per superblock, over the sub-blocks' sums of x (both
+// as three bf16 pieces).  The result is within three times the bound of fp32 sums of x w.
 //
 // A wave owns 16 columns: lane l holds column l % 16 and, of every sub-block, the values
 // 8 (l / 16) .. + 7.  Read straight from memory in that layout a superblock takes 5 loads that
@@ -19,10 +20,12 @@
 // workgroup on other columns share the staged x; KG groups of them split K for
 // narrow outputs.
 //
-// fp16 x, Q4_K: 1 x 151936 x 4096 (350 MB) 136 us on decoded weights -> 67 (5.2 TB/s); 1 x
-// 37888 x 3584 29.5 -> 22.5 us, 8 x 37888 x 3584 59 -> 27.  With the quants read in that
-// layout straight from memory the first took 119 us, with fp16 conversions instead of
-// subnormals 74, and with every LDS read draining the transfers (see u32x2) 96.
+// fp16 x, Q4_K: 1 x 151936 x 4096 (350 MB) 136 us on decoded weights -> 82 (4.3 TB/s); 1 x
+// 37888 x 3584 26.4 -> 22.8 us, 8 x 37888 x 3584 56 -> 29.2.  160 VALU instructions per
+// superblock of a wave's 16 columns, 2.5 per weight; with c_j = 0 (no centres: the bound then lies over the two parts, however
+// they cancel) the three take 73, 21.0 and 26.5 us; with a subtraction of c_j and a
+// multiply-add per sub-block 85, 23.6 and 30.5.  bf16 x, 2 x 37888 x 3584: 30.4 us, 34.6 with the
+// subtraction in fp32 after the conversion.
 //
 // Infinities and NaN: outputs that come out non-finite are recomputed weight by weight, as
 // in kq_gemm.hip.
@@ -92,21 +95,16 @@ struct KvRaw<NVF_Q4_K, LAYOUT> {
     }
   }
   static constexpr float kOdd = LAYOUT == NVF_QK_LAYOUT_GGML ? 0x1p20f : 0x1p24f;  // odd sub-blocks' 1 / unit
+  static constexpr float kTop = 15.0f;                                             // the largest quant
   __device__ __forceinline__ float d() const { return half_bits_to_f32(hdr[0] & 0xffffu); }
   __device__ __forceinline__ float dmin() const { return half_bits_to_f32(hdr[0] >> 16); }
-  // the eight 6-bit scales and minima, one per byte
-  __device__ __forceinline__ void tables(uint32_t* sc, uint32_t* mn) const {
-    sc[0] = hdr[1] & 0x3f3f3f3fu;
-    mn[0] = hdr[2] & 0x3f3f3f3fu;
-    sc[1] = (hdr[3] & 0x0f0f0f0fu) | ((hdr[1] >> 2) & 0x30303030u);
-    mn[1] = ((hdr[3] >> 4) & 0x0f0f0f0fu) | ((hdr[2] >> 2) & 0x30303030u);
-  }
 };
 
 template <int LAYOUT>
 struct KvRaw<NVF_Q5_K, LAYOUT> : KvRaw<NVF_Q4_K, NVF_QK_LAYOUT_GGML> {
   using Base = KvRaw<NVF_Q4_K, NVF_QK_LAYOUT_GGML>;
   static constexpr int kBlock = 176;
+  static constexpr float kTop = 31.0f;
   u32x2 h;
   __device__ __forceinline__ void load(const uint8_t* blk, int g) {
     hdr = ld16(blk);
@@ -134,29 +132,63 @@ struct KvRaw<NVF_Q5_K, LAYOUT> : KvRaw<NVF_Q4_K, NVF_QK_LAYOUT_GGML> {
   }
 };
 
-// The quants 8 g .. + 7 of sub-block s as 16-bit operands, and 1 / their unit.
+// Sub-block s's quants 8 g .. + 7 as 16-bit operands.  sub is what kv_sub made of the sub-block.
+// fp16: sc (q - c) 2^-14 by one exact multiply-add of the subnormal q (at most 11 bits).
 template <typename Raw>
-__device__ __forceinline__ u32x4 kv_operand(const Raw& r, int s, int g, float& unit, _Float16) {
-  unit = (s & 1) ? Raw::kOdd : 0x1p24f;
-  return r.halves(s, g);
+__device__ __forceinline__ u32x4 kv_operand(const Raw& r, int s, int g, uint32_t sub, _Float16) {
+  const f16x2 m = __builtin_bit_cast(f16x2, sub);
+  u32x4 p = r.halves(s, g);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t w = p[i];
+    p[i] = __builtin_bit_cast(
+        uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, w), f16x2{m[0], m[0]}, f16x2{m[1], m[1]}));
+  }
+  return p;
 }
+// The multiplier and the addend (exact in fp16); q's unit is 1 / kOdd in odd sub-blocks.
 template <typename Raw>
-__device__ __forceinline__ u32x4 kv_operand(const Raw& r, int s, int g, float& unit, __bf16) {
-  unit = 1.0f;
+__device__ __forceinline__ uint32_t kv_sub(float sc, float c, bool odd, _Float16) {
+  const float mul = odd ? 0x1p-14f * Raw::kOdd : 1024.0f;
+  const f16x2 m = {(_Float16)(mul * sc), (_Float16)(-0x1p-14f * sc * c)};
+  return __builtin_bit_cast(uint32_t, m);
+}
+// bf16: q - c (the scale would take a second operand)
+template <typename Raw>
+__device__ __forceinline__ u32x4 kv_operand(const Raw& r, int s, int g, uint32_t sub, __bf16) {
   uint32_t b[2];
   r.bytes(s, g, b);
+  // four weights at a time as signed bytes: 128 + q - c leaves no borrow, then the top bit flips
+#pragma unroll
+  for (int i = 0; i < 2; ++i) b[i] = (b[i] + sub) ^ 0x80808080u;
   u32x4 p;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {  // at most 5 significant bits: the upper halves of the fp32 values
-    const float v0 = (float)byte_of(b[i >> 1], 2 * (i & 1)), v1 = (float)byte_of(b[i >> 1], 2 * (i & 1) + 1);
+    const float v0 = sbyte(b[i >> 1], 2 * (i & 1)), v1 = sbyte(b[i >> 1], 2 * (i & 1) + 1);
     p[i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, v1), __builtin_bit_cast(uint32_t, v0), 0x07060302u);
   }
   return p;
 }
+template <typename Raw>
+__device__ __forceinline__ uint32_t kv_sub(float, float c, bool, __bf16) {
+  const uint32_t b = (uint32_t)c;
+  return 0x80808080u - b * 0x01010101u;
+}
+
+// v of the 16-lane group i in o[i], in every group.
+__device__ __forceinline__ void kv_gather(uint32_t v, uint32_t* o) {
+  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);              // groups 0 0 2 2, 1 1 3 3
+  const auto a = __builtin_amdgcn_permlane32_swap(r[0], r[0], false, false);        // 0 0 0 0, 2 2 2 2
+  const auto b = __builtin_amdgcn_permlane32_swap(r[1], r[1], false, false);        // 1 1 1 1, 3 3 3 3
+  o[0] = a[0];
+  o[1] = b[0];
+  o[2] = a[1];
+  o[3] = b[1];
+}
 
 // x as staged: XP planes of 16-bit values (fp32: three exact bf16 pieces), rows of a
 // superblock 528 bytes apart (the 16 rows of a read phase on distinct banks), then the
-// sub-blocks' sums as three bf16 pieces, [row][piece][8].
+// sub-blocks' sums' bf16 pieces, [row][8 j][x0 x0 x0 x1 x1 x2 0 0], rows 144 bytes apart.
 template <typename TX>
 struct KvX {
   using T = TX;
@@ -167,10 +199,10 @@ struct KvX<float> {
   using T = __bf16;
   static constexpr int kPlanes = 3;
 };
-constexpr int kKvRow = 528, kKvZero = 16;  // kKvZero bytes of zeros lead the LDS
+constexpr int kKvRow = 528, kKvSums = 144;
 template <typename TX>
 constexpr int kv_sb_bytes(int m) {
-  return m * (KvX<TX>::kPlanes * kKvRow + 48);
+  return m * (KvX<TX>::kPlanes * kKvRow + kKvSums);
 }
 
 // A weight stage in LDS: one superblock of 16 columns, column after column.  A column is 9 or
@@ -202,8 +234,8 @@ __global__ __launch_bounds__(WC* KG * 64) __attribute__((amdgpu_waves_per_eu(2, 
   const int per = (nsb + KG - 1) / KG;  // superblocks per K group
   const int sb0 = kg * per, cnt = nsb - sb0 < per ? nsb - sb0 : per;    // (cnt may be <= 0)
   const int sbb = kv_sb_bytes<TX>(m);
-  uint8_t* const ring = lds + kKvZero + wave * (kKvStages * Stage::kBytes);
-  uint8_t* const xl = lds + kKvZero + WC * KG * (kKvStages * Stage::kBytes) + kg * chunk * sbb;
+  uint8_t* const ring = lds + wave * (kKvStages * Stage::kBytes);
+  uint8_t* const xl = lds + WC * KG * (kKvStages * Stage::kBytes) + kg * chunk * sbb;
 
   // this lane's units of a stage; a column past n falls outside the resource and reads zero
   const int64_t row_bytes = (int64_t)nsb * Raw::kBlock;
@@ -225,7 +257,6 @@ __global__ __launch_bounds__(WC* KG * 64) __attribute__((amdgpu_waves_per_eu(2, 
   };
 #pragma unroll
   for (int st = 0; st < kKvStages - 1; ++st) issue(st, st);
-  if (threadIdx.x < kKvZero / 4) reinterpret_cast<uint32_t*>(lds)[threadIdx.x] = 0;
 
   // stages x of superblocks [i, i + chunk) of this group
   auto stage = [&](int i) {
@@ -256,13 +287,10 @@ __global__ __launch_bounds__(WC* KG * 64) __attribute__((amdgpu_waves_per_eu(2, 
       for (int e = 0; e < 8; ++e) sum += v[e];
       sum = group_sum<4>(sum);
       if ((ch & 3) == 0) {
-        const uint32_t h = __builtin_bit_cast(uint32_t, sum) & 0xffff0000u;
-        const float r1 = sum - __builtin_bit_cast(float, h);
-        const __bf16 b1 = (__bf16)r1, b2 = (__bf16)(r1 - (float)b1);
-        uint16_t* xs = reinterpret_cast<uint16_t*>(xl + s * sbb + XP * m * kKvRow + r * 48) + (ch >> 2);
-        xs[0] = (uint16_t)(h >> 16);
-        xs[8] = __builtin_bit_cast(uint16_t, b1);
-        xs[16] = __builtin_bit_cast(uint16_t, b2);
+        uint32_t pc[3];
+        bf16_pieces(sum, pc);
+        st16(xl + s * sbb + XP * m * kKvRow + r * kKvSums + 4 * ch,
+             u32x4{pc[0] | pc[0] << 16, pc[0] | pc[1] << 16, pc[1] | pc[2] << 16, 0u});
       }
     }
   };
@@ -270,36 +298,48 @@ __global__ __launch_bounds__(WC* KG * 64) __attribute__((amdgpu_waves_per_eu(2, 
   // Row r of x is operand row 4 (r % 4) + r / 4, so that lane group g's results e < NE are
   // rows g + 4 e: up to 4 NE rows cost NE multiply-adds per sub-block.  Operand rows of no
   // row of x repeat row 0; their results are not stored.
-  float tot[NE] = {};
+  f32x4 tot = {};
   const int xr = (c >> 2) + 4 * (c & 3), xrow = xr < m ? xr : 0;
   const uint8_t* const xa = xl + xrow * kKvRow + 16 * g;
-  const uint8_t* const xs = xl + XP * m * kKvRow + xrow * 48 + 16 * g;
+  const uint8_t* const xs = xl + XP * m * kKvRow + xrow * kKvSums + 32 * g;
   auto compute = [&](const Raw& r, int s) {  // superblock s of the staged chunk
     const uint8_t* xb = xa + s * sbb;
     const float d = r.d();
     uint32_t sc[2], mn[2];
-    r.tables(sc, mn);
+    q4k_tables(r.hdr, sc, mn);
+    // lane group g finds the centres of sub-blocks 2 g and 2 g + 1 and holds their remainders
+    // as [r0 r1 r2 r0 r1 r0 0 0]
+    const uint32_t sg = (g < 2 ? sc[0] : sc[1]) >> (16 * (g & 1)), mg = (g < 2 ? mn[0] : mn[1]) >> (16 * (g & 1));
+    uint32_t sub[2][4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float unit;
-      const u32x4 w = kv_operand(r, j, g, unit, T{});
-      f32x4 a = {};
-#pragma unroll
-      for (int p = XP - 1; p >= 0; --p) a = mfma16x16(ld16(xb + p * m * kKvRow + 64 * j), w, a, T{});
-      const float sj = (d * unit) * (float)byte_of(sc[j >> 2], j & 3);
-#pragma unroll
-      for (int e = 0; e < NE; ++e) tot[e] = fmaf(sj, a[e], tot[e]);
+    for (int i = 0; i < 2; ++i) {
+      const float sf = (float)byte_of(sg, i), p = d * sf, o = r.dmin() * (float)byte_of(mg, i);
+      const float q0 = kq_centre(p, o, Raw::kTop);
+      kv_gather(kv_sub<Raw>(sf, q0, i == 1, T{}), sub[i]);
+      uint32_t pc[3];
+      bf16_pieces(fmaf(p, q0, -o), pc);
+      const u32x4 rb = {pc[0] | pc[1] << 16, pc[2] | pc[0] << 16, pc[1] | pc[0] << 16, 0u};
+      tot = mfma16x16(ld16(xs + s * sbb + 16 * i), rb, tot, __bf16{});
     }
-    u32x4 mb;  // m_j in bf16 (6 bits)
+    if constexpr (__is_same(T, _Float16)) {  // the operands hold the scales
+      f32x4 a[2] = {};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float m0 = (float)byte_of(mn[i >> 1], 2 * (i & 1)), m1 = (float)byte_of(mn[i >> 1], 2 * (i & 1) + 1);
-      mb[i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, m1), __builtin_bit_cast(uint32_t, m0), 0x07060302u);
+      for (int j = 0; j < 8; ++j)
+        a[j & 1] = mfma16x16(ld16(xb + 64 * j), kv_operand(r, j, g, sub[j & 1][j >> 1], T{}), a[j & 1], T{});
+#pragma unroll
+      for (int e = 0; e < NE; ++e) tot[e] = fmaf(d * 0x1p14f, a[0][e] + a[1][e], tot[e]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const u32x4 w = kv_operand(r, j, g, sub[j & 1][j >> 1], T{});
+        f32x4 a = {};
+#pragma unroll
+        for (int p = XP - 1; p >= 0; --p) a = mfma16x16(ld16(xb + p * m * kKvRow + 64 * j), w, a, T{});
+        const float sj = d * (float)byte_of(sc[j >> 2], j & 3);
+#pragma unroll
+        for (int e = 0; e < NE; ++e) tot[e] = fmaf(sj, a[e], tot[e]);
+      }
     }
-    const f32x4 mm = mfma16x16(ld16(g < 3 ? xs + s * sbb : lds), mb, f32x4{}, __bf16{});
-    const float dm = -r.dmin();
-#pragma unroll
-    for (int e = 0; e < NE; ++e) tot[e] = fmaf(dm, mm[e], tot[e]);
   };
 
   // a barrier that leaves the weights' transfers in flight (a workgroup fence would drain them)
@@ -378,7 +418,7 @@ constexpr int kKvLds = 160 * 1024;
 template <typename TX, int BLOCK>
 int kv_lds(int m, int waves, int kg, int chunk) {
   const int part = (waves - waves / kg) * 64 * 16;
-  const int bytes = kKvZero + waves * kKvStages * KvStage<BLOCK>::kBytes + kg * chunk * kv_sb_bytes<TX>(m);
+  const int bytes = waves * kKvStages * KvStage<BLOCK>::kBytes + kg * chunk * kv_sb_bytes<TX>(m);
   return bytes > part ? bytes : part;
 }
 
@@ -388,7 +428,7 @@ int launch_kv(const TX* x, const uint8_t* w, TO* out, int64_t m, int64_t n, int6
   // x: the group's whole K where it is small, else chunks of about 16 KB per workgroup (three
   // workgroups of four waves per CU)
   const int per = ((int)(k >> 8) + KG - 1) / KG;
-  const int room = kKvLds - kKvZero - WC * KG * kKvStages * KvStage<kBlock>::kBytes;
+  const int room = kKvLds - WC * KG * kKvStages * KvStage<kBlock>::kBytes;
   const int most = ((room < 16 * 1024 ? room : 16 * 1024) / KG) / kv_sb_bytes<TX>((int)m);
   const int chunk = most < 1 ? 1 : most < per ? most : per;
   const int lds = kv_lds<TX, kBlock>((int)m, WC * KG, KG, chunk);

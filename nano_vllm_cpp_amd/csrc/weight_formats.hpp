@@ -104,6 +104,33 @@ __device__ __forceinline__ void q4k_sm(uint32_t h1, uint32_t h2, uint32_t h3, in
   }
 }
 
+// The eight 6-bit scales and minima of a Q4_K / Q5_K superblock's header, one per byte.
+__device__ __forceinline__ void q4k_tables(const u32x4 hdr, uint32_t* sc, uint32_t* mn) {
+  sc[0] = hdr[1] & 0x3f3f3f3fu;
+  mn[0] = hdr[2] & 0x3f3f3f3fu;
+  sc[1] = (hdr[3] & 0x0f0f0f0fu) | ((hdr[1] >> 2) & 0x30303030u);
+  mn[1] = ((hdr[3] >> 4) & 0x0f0f0f0fu) | ((hdr[2] >> 2) & 0x30303030u);
+}
+
+// The centre of a Q4_K / Q5_K sub-block with p = d sc and o = dmin mn: the quant q0 of 0 .. top
+// nearest to o / p.  Around it a weight p q - o is p (q - q0) + r with r = p q0 - o, and neither
+// part is larger than twice the weight (|r| <= |p| / 2, or q0 = 0 or top and both parts have one
+// sign): sums of the parts round no worse than sums of the weights, however p q and o cancel.
+// (p = 0, or no number at all: any q0 in the range will do, 0 here.)
+__device__ __forceinline__ float kq_centre(float p, float o, float top) {
+  return __builtin_amdgcn_fmed3f(__builtin_rintf(o * __builtin_amdgcn_rcpf(p)), 0.0f, top);
+}
+
+// The bits of v as three bf16 pieces (the first truncated).
+__device__ __forceinline__ void bf16_pieces(float v, uint32_t* p) {
+  const uint32_t h = __builtin_bit_cast(uint32_t, v) & 0xffff0000u;
+  const float r1 = v - __builtin_bit_cast(float, h);
+  const __bf16 b1 = (__bf16)r1, b2 = (__bf16)(r1 - (float)b1);
+  p[0] = h >> 16;
+  p[1] = __builtin_bit_cast(uint16_t, b1);
+  p[2] = __builtin_bit_cast(uint16_t, b2);
+}
+
 template <int N, int LAYOUT>
 struct Q4K {  // 144-byte superblocks; N consecutive outputs share one group j = i >> 5
   const uint8_t* wq;

@@ -152,3 +152,44 @@ def test_kquant_non_finite_operands(gpu, kind, layout, dt, m):
     assert (np.isposinf(got) == np.isposinf(want32)).all() and (np.isneginf(got) == np.isneginf(want32)).all()
     fin = np.isfinite(want32)
     assert np.allclose(got[fin], want32[fin], rtol=1e-4, atol=1e-3 * np.abs(want32[fin & (np.abs(want32) < 1e6)]).max())
+
+
+def cancelling_weights(r, n, k, kind, layout):
+    """Q4_K / Q5_K superblocks whose scale and offset parts cancel: in every sub-block one quant
+    q0 gives exactly 0 (every second superblock: almost 0), and all weights but one in every
+    third superblock hold it."""
+    nb = n * k // 256
+    sc = r.integers(1, 13, (nb, 8))
+    q0 = r.integers(1, np.minimum(16 if kind == 12 else 32, 63 // sc + 1))
+    q = np.repeat(q0[..., None], 32, 2)
+    some = np.arange(0, nb, 3)
+    q[some, r.integers(0, 8, some.size), r.integers(0, 32, some.size)] = r.integers(0, 16 if kind == 12 else 32, some.size)
+    d = r.uniform(1e-3, 1e-2, nb).astype(np.float16)
+    dmin = np.where(np.arange(nb) % 2, np.nextafter(d, np.float16(1)), d)
+    lo = (q & 15).astype(np.uint8)
+    if layout == H.GGML:
+        ql = (lo[:, 0::2] | lo[:, 1::2] << 4).reshape(nb, 128)
+    else:
+        ql = (lo[..., :16] | lo[..., 16:] << 4).reshape(nb, 128)
+    parts = [d.view(np.uint8).reshape(nb, 2), dmin.view(np.uint8).reshape(nb, 2), H.pack_q4k_scales(sc, sc * q0)]
+    if kind == 13:
+        parts.append(((q >> 4) << np.arange(8)[:, None]).sum(1).astype(np.uint8))
+    return np.concatenate(parts + [ql], 1).reshape(-1)
+
+
+@pytest.mark.parametrize("kind,layout", KQ[:3], ids=KQ_IDS[:3])
+@pytest.mark.parametrize("dt", [H.F16, H.BF16, H.F32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("m,n,k", [(1, 16400, 512), (4, 24, 8192), (13, 16400, 256), (70, 300, 768), (200, 130, 2048)])
+def test_kquant_scale_and_offset_cancel(gpu, kind, layout, dt, m, n, k):
+    """x of one sign on weights that are differences of large parts.  Around the quant q0
+    nearest to dmin m / (d sc) a weight is w = d sc (q - q0) + r with |d sc (q - q0)| <= 2 |w| and
+    |r| <= |w|, so sums of the two parts stay within three times the bound of sums of x w."""
+    if dt == H.F32 and m > 16:
+        pytest.skip("fp32 rows beyond the decode product take the tile kernel of test_gpu_dense_gemm.py")
+    r = H.rng(31 * kind + m)
+    x, w = H.gen_act(r, (m, k), dt, 1.0, 0.1), cancelling_weights(r, n, k, kind, layout)
+    want, err = kq_oracle(x, dt, w, kind, layout, m, n, k)
+    print(f"[case] kq cancel {kind}/{layout} {m}x{n}x{k} dt={dt}", flush=True)
+    got = ops.matmul(H.to_dev(x, gpu, dt), H.to_dev(w, gpu), n, kind, qk_layout=layout, out_dtype=torch.float32)
+    off = np.abs(got.double().cpu().numpy() - want)
+    assert (off <= 3 * err).all(), float((off / err).max())
