@@ -27,10 +27,12 @@
 // multiply-add per sub-block 85, 23.6 and 30.5.  bf16 x, 2 x 37888 x 3584: 30.4 us, 34.6 with the
 // subtraction in fp32 after the conversion.
 //
-// Infinities and NaN: outputs that come out non-finite are recomputed weight by weight, as
-// in kq_gemm.hip.
+// Infinities and NaN: sums that come out non-finite are made again from the decoded weights,
+// as in kq_gemm.hip (8 x 37888 x 3584, every activation NaN: 1040 us one
+// output after the other, 127 so).
 
 #include <mutex>
+#include <type_traits>
 
 #include "gemm16.hpp"
 #include "gemm_tile.hpp"
@@ -374,7 +376,40 @@ __global__ __launch_bounds__(WC* KG * 64) __attribute__((amdgpu_waves_per_eu(2, 
   }
   wait_vm<0>();
 
-  // lane l, value e: row l / 16 + 4 e, column l % 16
+  // lane l, value e: row l / 16 + 4 e, column l % 16.  Sums that came out infinite or NaN, again
+  // on the fp32 matrix cores (v_mfma_f32_16x16x4: value i of the four lane groups at a time).
+  const int64_t col = col0 + c;
+  bool bad = false;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) bad = bad || (g + 4 * e < m && col < n && !__builtin_isfinite(tot[e]));
+  if (__any(bad)) {
+    const Table<8, TX> xt{x};
+    using Plain = std::conditional_t<KIND == NVF_Q4_K, Q4K<8, LAYOUT>, Q5K<8>>;
+    const Plain wt{wq};
+    const int64_t x0 = (int64_t)xrow * k + 8 * g, w0 = (col < n ? col : n - 1) * k + 8 * g;
+    f32x4 v = {};
+#pragma unroll 1
+    for (int64_t i = (int64_t)sb0 * 256; i < (int64_t)(sb0 + cnt) * 256; i += 128) {
+      typename Table<8, TX>::Raw xr4[4];
+      typename Plain::Raw wr4[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {  // the loads of four steps go out together
+        xr4[u] = xt.load(x0 + i + 32 * u);
+        wr4[u] = wt.load(w0 + i + 32 * u);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        float xv[8], wv[8];
+        xt.decode(xr4[u], xv);
+        wt.decode(wr4[u], wv);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[q], wv[q], v, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+      if (!__builtin_isfinite(tot[e])) tot[e] = v[e];
+  }
   if constexpr (KG > 1) {  // the K groups' sums, in group order
     __syncthreads();
     float* part = reinterpret_cast<float*>(lds);
@@ -388,29 +423,10 @@ __global__ __launch_bounds__(WC* KG * 64) __attribute__((amdgpu_waves_per_eu(2, 
 #pragma unroll
       for (int e = 0; e < NE; ++e) tot[e] += part[(((q - 1) * WC + wc) * NE + e) * 64 + lane];
   }
-  const int64_t col = col0 + c;
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int r = g + 4 * e;
-    if (r >= m || col >= n) continue;
-    float v = tot[e];
-    if (!__builtin_isfinite(v)) {
-      v = 0.0f;
-#pragma unroll 1
-      for (int64_t i = 0; i < k; i += 4) {
-        float wv[4];
-        if constexpr (KIND == NVF_Q4_K) {
-          const Q4K<4, LAYOUT> w{wq};
-          w.decode(w.load(col * k + i), wv);
-        } else {
-          const Q5K<4> w{wq};
-          w.decode(w.load(col * k + i), wv);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v = fmaf(to_f32(x[(int64_t)r * k + i + q]), wv[q], v);
-      }
-    }
-    out[(int64_t)r * n + col] = from_f32<TO>(v);
+    if (r < m && col < n) out[(int64_t)r * n + col] = from_f32<TO>(tot[e]);
   }
 }
 

@@ -193,3 +193,26 @@ def test_kquant_scale_and_offset_cancel(gpu, kind, layout, dt, m, n, k):
     got = ops.matmul(H.to_dev(x, gpu, dt), H.to_dev(w, gpu), n, kind, qk_layout=layout, out_dtype=torch.float32)
     off = np.abs(got.double().cpu().numpy() - want)
     assert (off <= 3 * err).all(), float((off / err).max())
+
+
+@pytest.mark.parametrize("m,n,k", [(1021, 4096, 3584), (8, 37888, 3584), (2, 3584, 18944)], ids=["prefill", "wide", "deep"])
+def test_kquant_time_on_nan_activations(gpu, m, n, k):
+    """Every output non-finite: they are made again on the fp32 matrix cores, at most 16 times (their
+    rate to the 16-bit ones') the work of the product, and not one after the other."""
+    w = H.to_dev(H.gen_weights(H.rng(5), n, k, 12), gpu)
+    x = torch.ones(m, k, dtype=torch.float16, device=gpu)
+
+    def time(v):
+        best = float("inf")
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            ops.matmul(v, w, n, 12)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    t0, t1 = time(x), time(torch.full_like(x, float("nan")))
+    print(f"[case] NaN {m}x{n}x{k}: {1e3 * t0:.1f} us finite, {1e3 * t1:.1f} us NaN", flush=True)
+    assert t1 < 16 * t0
