@@ -551,13 +551,23 @@ __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(2))
     const KqPlain<KIND, LAYOUT> ws{wq};
     const int64_t x0 = (r0 + lr < m ? r0 + lr : m - 1) * k + 8 * half, w0 = (c < n ? c : n - 1) * k + 8 * half;
     f32x16 v = f32x16{};
-#pragma unroll 2
-    for (int64_t e = 0; e < k; e += 16) {
-      float xv[8], wv[8];
-      xs.decode(xs.load(x0 + e), xv);
-      ws.decode(ws.load(w0 + e), wv);
+#pragma unroll 1
+    for (int64_t e = 0; e < k; e += 32) {  // the loads of two steps go out together
+      typename Table<8, T>::Raw xr[2];
+      typename KqPlain<KIND, LAYOUT>::Raw wr[2];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[i], wv[i], v, 0, 0, 0);
+      for (int u = 0; u < 2; ++u) {
+        xr[u] = xs.load(x0 + e + 16 * u);
+        wr[u] = ws.load(w0 + e + 16 * u);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        float xv[8], wv[8];
+        xs.decode(xr[u], xv);
+        ws.decode(wr[u], wv);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[i], wv[i], v, 0, 0, 0);
+      }
     }
 #pragma unroll
     for (int j = 0; j < 16; ++j)
