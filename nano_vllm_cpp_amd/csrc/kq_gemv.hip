@@ -432,11 +432,31 @@ __global__ __launch_bounds__(WC* KG * 64) __attribute__((amdgpu_waves_per_eu(2, 
 
 constexpr int kKvLds = 160 * 1024;
 template <typename TX, int BLOCK>
-int kv_lds(int m, int waves, int kg, int chunk) {
-  const int part = (waves - waves / kg) * 64 * 16;
-  const int bytes = waves * kKvStages * KvStage<BLOCK>::kBytes + kg * chunk * kv_sb_bytes<TX>(m);
-  return bytes > part ? bytes : part;
+int kv_lds(int m, int waves, int kg, int chunk) {  // the rings and x; the groups' partial sums reuse the rings
+  static_assert(KvStage<BLOCK>::kBytes * kKvStages >= 64 * 16, "partial sums");
+  return waves * kKvStages * KvStage<BLOCK>::kBytes + kg * chunk * kv_sb_bytes<TX>(m);
 }
+
+// (A function per kernel, so that each has a flag of its own: the kernels are of one type.)
+template <typename TX, int KIND, int LAYOUT, typename TO, int WC, int KG, int NE>
+int launch_kv_kernel(const TX* x, const uint8_t* w, TO* out, int m, int64_t n, int64_t k, int chunk, int lds,
+                     hipStream_t st) {
+  auto kern = kq_gemv_kernel<TX, KIND, LAYOUT, TO, WC, KG, NE>;
+  static std::once_flag attr_once;
+  static hipError_t attr = hipSuccess;
+  std::call_once(attr_once, [&] {
+    attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kKvLds);
+  });
+  if (attr != hipSuccess)
+    return fail(NVF_ERR_LAUNCH, "dense_gemv (K-quant): %d bytes of LDS: %s", kKvLds, hipGetErrorString(attr));
+  kern<<<dim3((unsigned)((n + 16 * WC - 1) / (16 * WC))), WC * KG * 64, lds, st>>>(x, w, out, m, n, k, chunk);
+  return launch_status("dense_gemv (K-quant)");
+}
+
+// Narrow outputs split K over the workgroup's 8 waves, where kq_gemv_wins sends up to 8 rows (fp32 x:
+// 4) here; x then fits the LDS (145 KB at most, 4 rows of fp32 x on Q5_K).
+template <typename TX>
+constexpr int kKvSplitRows = sizeof(TX) == 4 ? 4 : 8;
 
 template <typename TX, int KIND, int LAYOUT, typename TO, int WC, int KG>
 int launch_kv(const TX* x, const uint8_t* w, TO* out, int64_t m, int64_t n, int64_t k, hipStream_t st) {
@@ -448,34 +468,19 @@ int launch_kv(const TX* x, const uint8_t* w, TO* out, int64_t m, int64_t n, int6
   const int most = ((room < 16 * 1024 ? room : 16 * 1024) / KG) / kv_sb_bytes<TX>((int)m);
   const int chunk = most < 1 ? 1 : most < per ? most : per;
   const int lds = kv_lds<TX, kBlock>((int)m, WC * KG, KG, chunk);
-  const dim3 grid((unsigned)((n + 16 * WC - 1) / (16 * WC)));
-  auto launch = [&](auto kern) {
-    static std::once_flag attr_once;
-    std::call_once(attr_once, [&] {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kKvLds);
-    });
-    kern<<<grid, WC * KG * 64, lds, st>>>(x, w, out, (int)m, n, k, chunk);
-  };
-  if (m <= 4)
-    launch(kq_gemv_kernel<TX, KIND, LAYOUT, TO, WC, KG, 1>);
-  else if (m <= 8)
-    launch(kq_gemv_kernel<TX, KIND, LAYOUT, TO, WC, KG, 2>);
-  else
-    launch(kq_gemv_kernel<TX, KIND, LAYOUT, TO, WC, KG, 4>);
-  return launch_status("dense_gemv (K-quant)");
+  constexpr int kMost = KG == 1 ? 16 : kKvSplitRows<TX>;
+  if constexpr (kMost > 8)
+    if (m > 8) return launch_kv_kernel<TX, KIND, LAYOUT, TO, WC, KG, 4>(x, w, out, (int)m, n, k, chunk, lds, st);
+  if constexpr (kMost > 4)
+    if (m > 4) return launch_kv_kernel<TX, KIND, LAYOUT, TO, WC, KG, 2>(x, w, out, (int)m, n, k, chunk, lds, st);
+  return launch_kv_kernel<TX, KIND, LAYOUT, TO, WC, KG, 1>(x, w, out, (int)m, n, k, chunk, lds, st);
 }
 
 template <typename TX, int KIND, int LAYOUT, typename TO>
 int launch_kv_split(const void* x, const uint8_t* w, void* out, int64_t m, int64_t n, int64_t k, hipStream_t st) {
-  constexpr int kBlock = KvRaw<KIND, LAYOUT>::kBlock;
   const TX* xp = static_cast<const TX*>(x);
   TO* op = static_cast<TO*>(out);
-  if (n < 16384) {
-    if (kv_lds<TX, kBlock>((int)m, 8, 8, 1) <= kKvLds)
-      return launch_kv<TX, KIND, LAYOUT, TO, 1, 8>(xp, w, op, m, n, k, st);
-    if (kv_lds<TX, kBlock>((int)m, 4, 4, 1) <= kKvLds)
-      return launch_kv<TX, KIND, LAYOUT, TO, 1, 4>(xp, w, op, m, n, k, st);
-  }
+  if (n < 16384 && m <= kKvSplitRows<TX>) return launch_kv<TX, KIND, LAYOUT, TO, 1, 8>(xp, w, op, m, n, k, st);
   return launch_kv<TX, KIND, LAYOUT, TO, 4, 1>(xp, w, op, m, n, k, st);
 }
 

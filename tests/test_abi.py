@@ -3,6 +3,7 @@ rejects bad arguments on the host (no GPU work is issued by these tests)."""
 from __future__ import annotations
 
 import re
+import subprocess
 from pathlib import Path
 
 import numpy as np
@@ -170,3 +171,13 @@ def test_decode_token_order(n):
         assert max(sums) - min(sums) <= int(kl.max())
     with pytest.raises(RuntimeError):
         ops._check(ops.lib().nvf_decode_token_order(kl.ctypes.data, -1, order.ctypes.data), "decode_token_order")
+
+
+def test_kquant_decode_kernels_opt_into_their_lds_each():
+    """Every kernel of the K-quant decode product has a once-flag of its own for the dynamic LDS it
+    asks for (one flag for several leaves all but the first called without it)."""
+    names = [ln.split()[-1] for ln in subprocess.run(["nm", str(ops.LIB_PATH)], capture_output=True, text=True,
+                                                     check=True).stdout.splitlines()]
+    kernels = [n for n in names if n.startswith("_ZN3nvf14kq_gemv_kernel")]
+    flags = [n for n in names if "launch_kv" in n and n.endswith("9attr_once")]
+    assert kernels and len(flags) == len(kernels)
