@@ -417,13 +417,15 @@ int nvf_paged_attention_ws(const void* q, void* out, const void* k_cache, const 
  * host: cu_seqlens_host [num_seqs + 1] (0, then each sequence's end; the last entry is
  * tokens), the packing that query_seq describes on the device (the reference's
  * cu_seqlens_q, include/nanovllm/context.hpp:8-25, built on the host by
- * ModelRunner::prepare_prefill, src/model_runner.cpp:43-128).  When no 128-token tile
- * holds more than 8 sequences, the launch for the tokens of such tiles is not made.
- * Results equal nvf_paged_attention_ws's.
+ * ModelRunner::prepare_prefill, src/model_runner.cpp:43-128).  128-token tiles of up to 8
+ * sequences stay on the prefill tiles as long as sequences with a few tokens there bring
+ * few keys; the tokens of the others are a second launch, made only where the packing
+ * allows such tiles.  Results equal nvf_paged_attention_ws's.
  * Contract: cu_seqlens_host must describe exactly the packing of query_seq (token t
- * belongs to sequence s iff cu_seqlens_host[s] <= t < cu_seqlens_host[s + 1]).  Only
- * its monotonicity and end points are checked; if it hides tiles of more than 8
- * sequences that query_seq has, the tokens of those tiles are left unwritten. */
+ * belongs to sequence s iff cu_seqlens_host[s] <= t < cu_seqlens_host[s + 1]), and
+ * query_key_len fits the block tables (at most block_size * max_blocks).  Only its
+ * monotonicity and end points are checked; tokens of tiles that it makes look like tiles
+ * of another kind may be left unwritten. */
 int nvf_paged_attention_seqs_ws(const void* q, void* out, const void* k_cache, const void* v_cache,
                                 const int32_t* query_seq, const int32_t* query_key_len, const int32_t* block_tables,
                                 const int32_t* cu_seqlens_host, int num_seqs, int64_t tokens, int q_heads,

@@ -120,35 +120,96 @@ struct Mfma16<_Float16> {
   }
 };
 
-// A tile's runs are its maximal stretches of consecutive tokens of one sequence.  A tile
-// of at most kFaMaxRuns runs is taken by the tile kernels, run after run: in a packed
-// prefill a tile that spans sequences holds one's tail and the next one's first keys, so
-// its further runs are short.  (Token by token on the decode kernels, whose chain over a
-// long context is serial, prompts of 4096, 3001, 2048 and 777 tokens took 132 us of 366 for
-// the 384 tokens of three tiles: 366 -> 263 us at fp16, fp32 prompts of 3072, 1531 and 700
-// 1070 -> 810; 32 prompts of 64 tokens 61 -> 17.)  A run costs about 3.5 us of latency, so a
-// crowded tile is better spread over the decode kernel's workgroups: 100 prompts of 20
-// tokens (7 runs) 60 -> 33 us, 300 of 8 (16 runs) 76 -> 68 but 400 of 5, whose last tile has
-// 16, 63 -> 114.  Every wave of a workgroup gets the same answer.
+// A tile's runs are its maximal stretches of consecutive tokens of one sequence.  The tile
+// kernels walk a tile's runs one after the other, each over its last token's keys; a tile
+// that they do not take goes to the decode kernels token by token, in a second launch.
+// A run of fewer than kThin tokens is thin: the tile kernel multiplies all 128 columns of each
+// 64-key chunk for its few, and its chunks are a chain that the decode kernel splits over four
+// waves.  A tile of up to kFaMaxRuns runs is taken if its thin runs' chunks sum to at most
+// kExtra, the longest of those that go on outside the tile apart (whatever tile holds the
+// sequence's other tokens takes as long).  So
+//   * the ends of packed prompts stay (4096, 3001, 2048 and 777 tokens at fp16, 384 of them in
+//     such tiles: 366 us with these on the decode kernels, 266 so; fp32 prompts of 3072, 1531
+//     and 700 tokens 1070 -> 815; 32 of 64 tokens 76 -> 27), and so do chunks of many tokens
+//     after cached keys (2 x 1500 after 4096: fp16 468 -> 370, fp32 3155 -> 2015);
+//   * a decode token over a long context packed with a prompt does not hold up its tile (7 at
+//     4096 keys and a prompt of 3000 tokens: fp16 795 us walked, 148 so; fp32 4785, 752).
+// 16-token chunks after 1024 keys (160 of them) take fp16 611 us on the decode kernels and 425
+// walked, fp32 1060 and 3450; 64-token chunks after 4096 keys (40) 1135 and 420, 3570 and 3370.
+// More than 8 short runs are better spread over the decode kernels' workgroups (400 prompts
+// of 5 tokens 63 us, 114 walked).  Every wave of a workgroup gets the same answer.
 constexpr int kFaMaxRuns = 8;
+template <typename T>
+struct FaTake {  // in tokens; in 64-key chunks
+  static constexpr int kThin = sizeof(T) == 2 ? 16 : 32, kExtra = sizeof(T) == 2 ? 8 : 2;
+};
 struct FaRuns {  // bit i: the tile's token i starts a run (token 0's bit is clear)
   uint64_t lo, hi;
-  __device__ __forceinline__ bool taken() const { return __popcll(lo) + __popcll(hi) < kFaMaxRuns; }
+  bool taken;
   // the first run start after token r, or the tile's end
   __device__ __forceinline__ int end_after(int r, int end) const {
     const uint64_t a = r < 63 ? lo >> (r + 1) << (r + 1) : 0;
     const uint64_t b = r < 64 ? hi : r < 127 ? hi >> (r - 63) << (r - 63) : 0;
     return a ? __builtin_ctzll(a) : b ? 64 + __builtin_ctzll(b) : end;
   }
+  // the start of token r's run
+  __device__ __forceinline__ int start_of(int r) const {
+    const uint64_t a = r < 63 ? lo & ((2ull << r) - 1) : lo;
+    const uint64_t b = r < 64 ? 0 : r < 127 ? hi & ((2ull << (r - 64)) - 1) : hi;
+    return b ? 127 - __builtin_clzll(b) : a ? 63 - __builtin_clzll(a) : 0;
+  }
 };
-__device__ __forceinline__ FaRuns fa_tile_runs(const int32_t* __restrict__ qseq, int64_t tokens, int64_t tile) {
+template <typename T>
+__device__ __forceinline__ FaRuns fa_tile_runs(const int32_t* __restrict__ qseq, const int32_t* __restrict__ qlen,
+                                               int64_t tokens, int64_t tile) {
   static_assert(kFaBq == 128, "two tokens per lane");
   const int lane = threadIdx.x & 63;
-  const int64_t t = tile * kFaBq + lane, last = tokens - 1;  // past the end: the last token again, no start
-  const int32_t a = qseq[t < last ? t : last], b = qseq[t + 64 < last ? t + 64 : last];
+  const int64_t t0 = tile * kFaBq, last = tokens - 1;  // past the end: the last token again, no start
+  const int end = tokens - t0 < kFaBq ? (int)(tokens - t0) : kFaBq;  // the tile's tokens
+  const int64_t ta = t0 + lane < last ? t0 + lane : last, tb = t0 + lane + 64 < last ? t0 + lane + 64 : last;
+  const int32_t a = qseq[ta], b = qseq[tb], la = qlen[ta], lb = qlen[tb];
+  const int32_t before = qseq[t0 > 0 ? t0 - 1 : 0], after = qseq[t0 + end < tokens ? t0 + end : last];
   const int32_t pa = __shfl_up(a, 1), pb = __shfl_up(b, 1);
-  const int32_t a63 = __builtin_amdgcn_readlane(a, 63);
-  return {__ballot(lane > 0 && a != pa), __ballot(b != (lane > 0 ? pb : a63))};
+  const int32_t a0 = __builtin_amdgcn_readlane(a, 0), a63 = __builtin_amdgcn_readlane(a, 63);
+  FaRuns r{__ballot(lane > 0 && a != pa), __ballot(b != (lane > 0 ? pb : a63)), true};
+  const int starts = __popcll(r.lo) + __popcll(r.hi);
+  if (starts == 0) return r;
+  if (starts >= kFaMaxRuns) {
+    r.taken = false;
+    return r;
+  }
+  // this lane's runs: the chunks of those that end at its tokens and are thin
+  const bool back = t0 > 0 && before == a0, on = t0 + end < tokens;
+  const int32_t b63 = __builtin_amdgcn_readlane(b, 63);  // the tile's last token's sequence, if the tile is full
+  float thin = 0.0f, outside = 0.0f;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int i = lane + 64 * h, len = h ? lb : la, first = r.start_of(i);
+    if (i >= end || r.end_after(i, end) != i + 1 || i + 1 - first >= FaTake<T>::kThin) continue;
+    const float c = len > 0 ? fminf((float)(((uint32_t)len + 63u) / 64u), 65536.0f) : 0.0f;
+    thin += c;
+    if ((first == 0 && back) || (i + 1 == end && on && after == b63)) outside = fmaxf(outside, c);
+  }
+  r.taken = wave_sum(thin) - wave_max(outside) <= (float)FaTake<T>::kExtra;  // whole numbers: exact
+  return r;
+}
+
+// Tiles that may not be taken, where the host knows the packing (n = 0: it does not); their
+// tokens are then the second launch, a workgroup per (token, kv head).  Up to kFaListMax: a
+// workgroup that only leaves costs about 3 ns, and a token's kv heads one after the other
+// save three of four such (32 prompts of 64 tokens: 27 us without the second launch, 57 with
+// it over 16 listed tiles, 33 over all tokens).
+constexpr int kFaListMax = 7;
+struct FaTileList {
+  int32_t n;
+  int32_t tile[kFaListMax];
+};
+// The second launch's token of this workgroup: of the listed tiles (workgroup = token, kv head),
+// or of all (past the batch: no token).
+__device__ __forceinline__ int64_t fa_listed_token(const FaTileList& list, int kv_heads) {
+  if (list.n == 0) return (int64_t)blockIdx.x;
+  const int x = (int)(blockIdx.x / kv_heads);
+  return (int64_t)list.tile[x / kFaBq] * kFaBq + x % kFaBq;
 }
 
 // This lane, from the hardware's count, opaque to the optimizer.
@@ -172,8 +233,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 :
   const int64_t tile = tiles - 1 - bid / q_heads;  // the longest tiles (latest positions) first
   const int h = (int)(bid % q_heads);
   const int64_t t0 = tile * kFaBq;
-  const FaRuns runs = fa_tile_runs(qseq, tokens, tile);
-  if (!runs.taken()) return;  // the whole workgroup: left to the decode kernel
+  const FaRuns runs = fa_tile_runs<T>(qseq, qlen, tokens, tile);
+  if (!runs.taken) return;  // the whole workgroup: left to the decode kernel
   const int kvh = h / (q_heads / kv_heads);
   const int64_t kv_stride = (int64_t)kv_heads * kFaHd;
   const int tend = tokens - t0 < kFaBq ? (int)(tokens - t0) : kFaBq;
@@ -481,8 +542,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   const int64_t tile = tiles - 1 - bid / q_heads;  // the longest tiles (latest positions) first
   const int h = (int)(bid % q_heads);
   const int64_t t0 = tile * kFaBq;
-  const FaRuns runs = fa_tile_runs(qseq, tokens, tile);
-  if (!runs.taken()) return;  // the whole workgroup: left to the decode kernel
+  const FaRuns runs = fa_tile_runs<float>(qseq, qlen, tokens, tile);
+  if (!runs.taken) return;  // the whole workgroup: left to the decode kernel
   const int kvh = h / (q_heads / kv_heads);
   const int64_t kv_stride = (int64_t)kv_heads * kFaHd;
   const int tend = tokens - t0 < kFaBq ? (int)(tokens - t0) : kFaBq;
@@ -775,7 +836,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
     const T* __restrict__ q, T* __restrict__ out, const T* __restrict__ kc, const T* __restrict__ vc,
     const int32_t* __restrict__ qseq, const int32_t* __restrict__ qlen, const int32_t* __restrict__ tables,
     int64_t tokens, int q_heads, int kv_heads, int bs, int max_blocks, float scale_log2, int64_t q_stride,
-    int split_keys, float* __restrict__ part, const int32_t* __restrict__ order) {
+    int split_keys, float* __restrict__ part, const int32_t* __restrict__ order, FaTileList list) {
   using M = Mfma16x16<T>;
   using v8 = typename M::v8;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -791,7 +852,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   // token's kv heads spread over the grid: 210 against 223 us for random lengths).
   const bool self_order = !SKIP && !SPLIT && !order && tokens <= kDecSelfOrderMax;
   const bool tok_major = !SKIP && (order || self_order);
-  const int64_t ti = SKIP ? (int64_t)blockIdx.x
+  const int64_t ti = SKIP ? fa_listed_token(list, kv_heads)
                      : tok_major ? (int64_t)blockIdx.x / kv_heads
                                  : (int64_t)blockIdx.x % tokens;
   int64_t t;
@@ -828,12 +889,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   }
   if (t < 0 || t >= tokens) return;  // an order entry outside the batch: nothing to compute (uniform)
   // workgroup-uniform: the whole workgroup leaves (fa_prefill_kernel's tile)
-  if (SKIP && fa_tile_runs(qseq, tokens, t / kFaBq).taken()) return;
-  // The tiles' second launch (SKIP) has one workgroup per token, so that its many
-  // exiting workgroups stay few, and walks the kv heads; otherwise the workgroup's
-  // kv head (one trip).
-  const int kvh0 = SKIP ? 0 : tok_major ? (int)(blockIdx.x % kv_heads) : (int)(blockIdx.x / tokens);
-  const int kvh1 = SKIP ? kv_heads : kvh0 + 1;
+  if (SKIP && fa_tile_runs<T>(qseq, qlen, tokens, t / kFaBq).taken) return;
+  // The tiles' second launch (SKIP) has one workgroup per (token, kv head) of the host's
+  // listed tiles; without a list, one per token, so that its many exiting workgroups stay few,
+  // and walks the kv heads.  Otherwise the workgroup's kv head (one trip).
+  const bool walk = SKIP && list.n == 0;
+  const int kvh0 = walk ? 0 : SKIP || tok_major ? (int)(blockIdx.x % kv_heads) : (int)(blockIdx.x / tokens);
+  const int kvh1 = walk ? kv_heads : kvh0 + 1;
   for (int kvh = kvh0; kvh < kvh1; ++kvh) {
     const int G = q_heads / kv_heads;
     const int col = lane & 15, g = lane >> 4;
@@ -1020,21 +1082,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
     const float* __restrict__ q, float* __restrict__ out, const float* __restrict__ kc, const float* __restrict__ vc,
     const int32_t* __restrict__ qseq, const int32_t* __restrict__ qlen, const int32_t* __restrict__ tables,
     int64_t tokens, int q_heads, int kv_heads, int bs, int max_blocks, float scale_log2, int64_t q_stride,
-    int split_keys, float* __restrict__ part, const int32_t* __restrict__ order) {
+    int split_keys, float* __restrict__ part, const int32_t* __restrict__ order, FaTileList list) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   __shared__ float merge[4][kDecMergeFloats];
   const bool tok_major = !SKIP && order;  // the workgroup's (token, kv head) as fa_decode_kernel's
-  const int64_t ti = SKIP ? (int64_t)blockIdx.x
+  const int64_t ti = SKIP ? fa_listed_token(list, kv_heads)
                      : tok_major ? (int64_t)blockIdx.x / kv_heads
                                  : (int64_t)blockIdx.x % tokens;
   const int64_t t = tok_major ? (int64_t)order[ti] : ti;
   if (t < 0 || t >= tokens) return;
   // workgroup-uniform: the whole workgroup leaves (fa_prefill_f32_kernel's tile)
-  if (SKIP && fa_tile_runs(qseq, tokens, t / kFaBq).taken()) return;
-  // as fa_decode_kernel: the tiles' second launch walks the kv heads per token
-  const int kvh0 = SKIP ? 0 : tok_major ? (int)(blockIdx.x % kv_heads) : (int)(blockIdx.x / tokens);
-  const int kvh1 = SKIP ? kv_heads : kvh0 + 1;
+  if (SKIP && fa_tile_runs<float>(qseq, qlen, tokens, t / kFaBq).taken) return;
+  const bool walk = SKIP && list.n == 0;  // as fa_decode_kernel
+  const int kvh0 = walk ? 0 : SKIP || tok_major ? (int)(blockIdx.x % kv_heads) : (int)(blockIdx.x / tokens);
+  const int kvh1 = walk ? kv_heads : kvh0 + 1;
   for (int kvh = kvh0; kvh < kvh1; ++kvh) {
     const int G = q_heads / kv_heads;
     const int col = lane & 15, g = lane >> 4;
@@ -1180,7 +1242,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_wave_kernel(
   if (gw >= tokens * q_heads) return;  // whole waves only; no workgroup barrier below
   const int64_t t = gw / q_heads;
   const int h = (int)(gw - t * q_heads);
-  if (skip_taken_tiles && fa_tile_runs(qseq, tokens, t / kFaBq).taken()) return;  // fa_prefill_kernel's
+  if (skip_taken_tiles && fa_tile_runs<T>(qseq, qlen, tokens, t / kFaBq).taken) return;  // fa_prefill_kernel's
   const int kvh = h / (q_heads / kv_heads);
   const int L = qlen[t];
   T* o = out + (t * q_heads + h) * hd;
@@ -1374,14 +1436,48 @@ void launch_attn_wave(const void* q, void* out, const void* kc, const void* vc, 
   }
 }
 
+// The tiles that fa_tile_runs may not take whatever their key counts (at most `keys`) are.
+template <typename T>
+FaTileList fa_doubtful_tiles(const int32_t* cu, int num_seqs, int64_t keys) {
+  FaTileList list{};
+  const int64_t most = (keys + 63) / 64;  // chunks of a run
+  int64_t tile = -1;
+  int runs = 0, thin = 0, outside = 0;  // the tile's runs so far; the thin ones that end in it, and that go on
+  const auto close = [&] {
+    const int64_t chunks = (thin + (outside > 1 ? outside - 1 : 0)) * most;
+    if (runs < 2 || list.n < 0 || (runs <= kFaMaxRuns && chunks <= FaTake<T>::kExtra)) return;
+    if (list.n == kFaListMax) list.n = -1;
+    else list.tile[list.n++] = (int32_t)tile;
+  };
+  const auto add = [&](int64_t at, int64_t n, bool goes_on) {  // a run of the tile that holds token at
+    if (at / kFaBq != tile) {
+      close();
+      tile = at / kFaBq;
+      runs = thin = outside = 0;
+    }
+    ++runs;
+    if (n < FaTake<T>::kThin) ++(goes_on ? outside : thin);
+  };
+  for (int s = 0; s < num_seqs; ++s) {  // a sequence's first tile and, if another, its last: those between are its own
+    const int64_t b = cu[s], e = cu[s + 1];
+    if (b == e) continue;
+    const int64_t first_end = std::min<int64_t>(e, (b / kFaBq + 1) * kFaBq), last = (e - 1) / kFaBq * kFaBq;
+    add(b, first_end - b, first_end < e);
+    if (last > b) add(last, e - last, true);
+  }
+  close();
+  return list;
+}
+
 template <typename T>
 int attention_dispatch(const void* q, void* out, const void* kc, const void* vc, const int32_t* qseq,
                        const int32_t* qlen, const int32_t* tables, int64_t tokens, int q_heads, int kv_heads, int hd,
                        int bs, int max_blocks, float scale, int64_t q_stride, int64_t max_query_len, void* ws,
-                       int64_t ws_bytes, hipStream_t st, bool taken = false, const int32_t* order = nullptr) {
-  // taken: no tile has more than kFaMaxRuns runs (counted on the host from the caller's
-  // cu_seqlens), so the tile kernel takes every token and the tiles' second launch,
-  // whose workgroups would all exit, is not made
+                       int64_t ws_bytes, hipStream_t st, const FaTileList* mixed = nullptr,
+                       const int32_t* order = nullptr) {
+  // mixed: the tiles that may not be taken, from the caller's cu_seqlens (n = -1: more than the
+  // list holds).  With none the tile kernel takes every token and the tiles' second launch,
+  // whose workgroups would all exit, is not made; else it is made for their tokens.
   constexpr int N = Pack<T>::N;
   if (tokens * kv_heads > INT32_MAX) return fail(NVF_ERR_INVALID, "paged_attention: too many tokens");
   const float sl = scale * 1.4426950408889634f;
@@ -1445,21 +1541,23 @@ int attention_dispatch(const void* q, void* out, const void* kc, const void* vc,
     const int rc = launch_status("paged_attention(tiles)");
     if (rc != NVF_OK) return rc;
   }
-  if (tiles && taken) {
+  if (tiles && mixed && mixed->n == 0) {
     if (!split) return NVF_OK;
     attn_split_combine_kernel<T><<<dim3((unsigned)tokens, (unsigned)q_heads), 256, 0, st>>>(part, ot, tokens,
                                                                                             q_heads, sp.nsplit);
     return launch_status("paged_attention(split merge)");
   }
   if (dec) {
-    // one workgroup per (token, kv head); for the tiles' second launch (SKIP), one
-    // per token walking the kv heads, since nearly all of its workgroups exit at once
-    const dim3 grid((unsigned)(tiles ? tokens : tokens * kv_heads), 1u, nz);
+    // one workgroup per (token, kv head); for the tiles' second launch (SKIP) without a list of
+    // tiles, one per token walking the kv heads, since nearly all of its workgroups exit at once
+    FaTileList list{};
+    if (tiles && mixed && mixed->n > 0) list = *mixed;
+    const dim3 grid((unsigned)(!tiles ? tokens * kv_heads : list.n ? list.n * kFaBq * kv_heads : tokens), 1u, nz);
     const int kk = split ? skeys : 0;
     float* pp = split ? part : nullptr;
 #define NVF_DEC_LAUNCH_ORD(KERN, LDS, ORD)                                                                     \
   KERN<<<grid, 256, LDS, st>>>(qt, ot, kt, vt, qseq, qlen, tables, tokens, q_heads, kv_heads, bs, max_blocks, sl, \
-                               q_stride, kk, pp, ORD)
+                               q_stride, kk, pp, ORD, list)
     if constexpr (sizeof(T) == 2) {
       static std::once_flag dec_once;
       std::call_once(dec_once, [] {
@@ -1554,8 +1652,8 @@ static int paged_attention_entry(const void* q, void* out, const void* k_cache, 
                                  const int32_t* query_seq, const int32_t* query_key_len, const int32_t* block_tables,
                                  int64_t tokens, int q_heads, int kv_heads, int head_dim, int block_size,
                                  int max_blocks, float scale, int64_t q_stride, int64_t max_query_len, void* workspace,
-                                 int64_t workspace_bytes, int dtype, void* stream, bool aligned,
-                                 const int32_t* order = nullptr) {
+                                 int64_t workspace_bytes, int dtype, void* stream,
+                                 const FaTileList* mixed = nullptr, const int32_t* order = nullptr) {
   if (!dtype_ok(dtype)) return fail(NVF_ERR_INVALID, "nvf_paged_attention: bad dtype %d", dtype);
   if (tokens < 0 || q_heads <= 0 || kv_heads <= 0 || head_dim <= 0 || block_size <= 0 || max_blocks <= 0)
     return fail(NVF_ERR_INVALID, "nvf_paged_attention: bad shape");
@@ -1575,7 +1673,7 @@ static int paged_attention_entry(const void* q, void* out, const void* k_cache, 
   NVF_DISPATCH_DTYPE(dtype, T, rc = attention_dispatch<T>(q, out, k_cache, v_cache, query_seq, query_key_len,
                                                          block_tables, tokens, q_heads, kv_heads, head_dim, block_size,
                                                          max_blocks, scale, q_stride, max_query_len, workspace,
-                                                         workspace_bytes, as_stream(stream), aligned, order));
+                                                         workspace_bytes, as_stream(stream), mixed, order));
   return rc;
 }
 
@@ -1586,7 +1684,7 @@ int nvf_paged_attention_ws(const void* q, void* out, const void* k_cache, const 
                            int64_t workspace_bytes, int dtype, void* stream) {
   return paged_attention_entry(q, out, k_cache, v_cache, query_seq, query_key_len, block_tables, tokens, q_heads,
                                kv_heads, head_dim, block_size, max_blocks, scale, q_stride, max_query_len, workspace,
-                               workspace_bytes, dtype, stream, false);
+                               workspace_bytes, dtype, stream);
 }
 
 int nvf_decode_token_order(const int32_t* key_len_host, int64_t tokens, int32_t* order_host) {
@@ -1617,7 +1715,7 @@ int nvf_paged_attention_order_ws(const void* q, void* out, const void* k_cache, 
   if (!token_order) return fail(NVF_ERR_INVALID, "nvf_paged_attention_order_ws: NULL token_order");
   return paged_attention_entry(q, out, k_cache, v_cache, query_seq, query_key_len, block_tables, tokens, q_heads,
                                kv_heads, head_dim, block_size, max_blocks, scale, q_stride, max_query_len, workspace,
-                               workspace_bytes, dtype, stream, false, token_order);
+                               workspace_bytes, dtype, stream, nullptr, token_order);
 }
 
 int nvf_paged_attention_seqs_ws(const void* q, void* out, const void* k_cache, const void* v_cache,
@@ -1631,20 +1729,14 @@ int nvf_paged_attention_seqs_ws(const void* q, void* out, const void* k_cache, c
   if (cu_seqlens_host[0] != 0 || cu_seqlens_host[num_seqs] != tokens)
     return fail(NVF_ERR_INVALID, "nvf_paged_attention_seqs_ws: cu_seqlens must run from 0 to tokens=%lld",
                 (long long)tokens);
-  bool taken = true;
-  int64_t tile = -1;  // the tile of the last sequence start inside a tile, and its runs so far
-  int runs = 1;
-  for (int s = 1; s <= num_seqs; ++s) {
+  for (int s = 1; s <= num_seqs; ++s)
     if (cu_seqlens_host[s] < cu_seqlens_host[s - 1])
       return fail(NVF_ERR_INVALID, "nvf_paged_attention_seqs_ws: cu_seqlens must not decrease");
-    if (s == num_seqs || cu_seqlens_host[s] == cu_seqlens_host[s - 1] || cu_seqlens_host[s] % kFaBq == 0) continue;
-    runs = cu_seqlens_host[s] / kFaBq == tile ? runs + 1 : 2;
-    tile = cu_seqlens_host[s] / kFaBq;
-    if (runs > kFaMaxRuns) taken = false;
-  }
+  FaTileList mixed{};
+  NVF_DISPATCH_DTYPE(dtype, T, mixed = fa_doubtful_tiles<T>(cu_seqlens_host, num_seqs, (int64_t)block_size * max_blocks));
   return paged_attention_entry(q, out, k_cache, v_cache, query_seq, query_key_len, block_tables, tokens, q_heads,
                                kv_heads, head_dim, block_size, max_blocks, scale, q_stride, max_query_len, workspace,
-                               workspace_bytes, dtype, stream, taken);
+                               workspace_bytes, dtype, stream, &mixed);
 }
 
 int nvf_paged_attention(const void* q, void* out, const void* k_cache, const void* v_cache, const int32_t* query_seq,
@@ -1725,7 +1817,7 @@ int nvf_paged_attention_noalloc(const void* q, void* out, const void* k_cache, c
   if (need > 0 && !(ws = scratch_ptr())) return NVF_ERR_LAUNCH;
   return paged_attention_entry(q, out, k_cache, v_cache, query_seq, query_key_len, block_tables, tokens, q_heads,
                                kv_heads, head_dim, block_size, max_blocks, scale, q_stride, max_query_len, ws, need,
-                               dtype, stream, false);
+                               dtype, stream);
 }
 
 // Drop-ins: include/nanovllm/hip_ops.hpp:22-28 / src/hip_ops.hip:724-744 (fp32 cache, null stream).

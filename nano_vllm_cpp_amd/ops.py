@@ -354,8 +354,8 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     give the library the workspace for split attention when the shape calls for
     it (little work over long contexts); False runs unsplit.  cu_seqlens: the
     batch's packing on the host ([seqs + 1] ints, 0 .. tokens), if the caller has it
-    (nvf_paged_attention_seqs_ws: no launch for crowded tiles when no 128-token tile
-    holds more than 8 sequences).  noalloc: nvf_paged_attention_noalloc (the
+    (nvf_paged_attention_seqs_ws: a second launch only where a 128-token tile may hold a
+    sequence of few tokens over many keys).  noalloc: nvf_paged_attention_noalloc (the
     split's partials in the library's static device scratch, no workspace
     allocated).  token_order: a device int32 [tokens] permutation of the tokens over the
     decode kernel's workgroups (decode_token_order; nvf_paged_attention_order_ws), results

@@ -624,3 +624,64 @@ def test_paged_attention_tiles_of_several_sequences(gpu, dt, ci):
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     host = ops.paged_attention(*args, bs, hd ** -0.5, split=split, cu_seqlens=cu)
     H.assert_bitexact(H.to_host(host), H.to_host(got), "host cu_seqlens vs device-only metadata")
+
+
+# (context, query) lengths of packed sequences: tiles that the tile kernels take and leave by the
+# keys of their runs, and the second launch over listed and over all tokens.
+MIXED_CASES = [
+    [(700, 1)] * 3 + [(300, 300)],                 # decode tokens ahead of a prompt
+    [(300, 300), (1500, 1), (64, 1), (700, 40)],   # and behind it, with a short chunk after cached keys
+    [(900, 16)] * 10,                              # 16 tokens per chunk of keys, 8 runs
+    [(400, 64)] * 6,                               # 64
+    [(200, 90), (1000, 140), (150, 100)],          # chunks after cached keys that go on in the next tile
+    [(500, 1), (200, 200)] * 40,                   # more such tiles than the list holds
+    [(2, 1)] * 6 + [(122, 122), (4100, 1)],        # the last token of a partial tile
+]
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=DT_IDS)
+@pytest.mark.parametrize("split", [False, True], ids=["whole", "split"])
+@pytest.mark.parametrize("ci", range(len(MIXED_CASES)))
+def test_paged_attention_prompts_packed_with_long_contexts(gpu, dt, split, ci):
+    """Against the oracle without the host's packing; with it, the same bits."""
+    ctx, lens = [c for c, _ in MIXED_CASES[ci]], [n for _, n in MIXED_CASES[ci]]
+    q_heads, kv_heads, hd, bs = 4, 2, 128, 64
+    b = H.make_paged(H.rng(1700 + 10 * ci + dt), ctx, lens, q_heads, kv_heads, hd, bs, dt)
+    exact, vmax = H.oracle_attention(b, q_heads, kv_heads, hd, bs, hd ** -0.5, dt)[1:]
+    args = [H.to_dev(b.q, gpu, dt), H.to_dev(b.k_cache, gpu, dt), H.to_dev(b.v_cache, gpu, dt),
+            H.to_dev(b.query_seq, gpu), H.to_dev(b.query_key_len, gpu), H.to_dev(b.block_tables, gpu)]
+    case(f"attention mixed {ci} split={split} dt={dt}")
+    got = ops.paged_attention(*args, bs, hd ** -0.5, split=split)
+    assert_attn(H.to_host(got), exact, vmax, dt, f"mixed {ci}")
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    host = ops.paged_attention(*args, bs, hd ** -0.5, split=split, cu_seqlens=cu)
+    H.assert_bitexact(H.to_host(host), H.to_host(got), "host cu_seqlens vs device-only metadata")
+
+
+@pytest.mark.parametrize("dt", [H.F32, H.F16], ids=["f32", "f16"])
+def test_paged_attention_time_of_decode_tokens_in_a_prompt(gpu, dt):
+    """Decode tokens over a long context packed with a prompt cost about what they cost alone: they
+    do not make the prompt's tiles walk their keys one after the other."""
+    q_heads, kv_heads, hd, bs = 28, 4, 128, 256
+    args = {}
+    for name, seqs in (("both", [(4096, 1)] * 7 + [(3000, 3000)]), ("prompt", [(3000, 3000)]), ("decode", [(4096, 1)] * 7)):
+        ctx, lens = [c for c, _ in seqs], [n for _, n in seqs]
+        b = H.make_paged(H.rng(3), ctx, lens, q_heads, kv_heads, hd, bs, dt)
+        args[name] = ([H.to_dev(b.q, gpu, dt), H.to_dev(b.k_cache, gpu, dt), H.to_dev(b.v_cache, gpu, dt),
+                       H.to_dev(b.query_seq, gpu), H.to_dev(b.query_key_len, gpu), H.to_dev(b.block_tables, gpu), bs,
+                       hd ** -0.5], np.concatenate([[0], np.cumsum(lens)]).astype(np.int32))
+
+    def time(name):
+        best = float("inf")
+        for _ in range(5):
+            a, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            ops.paged_attention(*args[name][0], cu_seqlens=args[name][1])
+            e.record()
+            e.synchronize()
+            best = min(best, a.elapsed_time(e))
+        return best
+
+    t = {name: time(name) for name in args}
+    case(f"decode tokens in a prompt dt={dt}: {t}")
+    assert t["both"] < 2 * (t["prompt"] + t["decode"])
