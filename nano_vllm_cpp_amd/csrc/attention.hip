@@ -219,8 +219,10 @@ __device__ __forceinline__ int fa_lane() {
   return lane;
 }
 
+// (Three waves per SIMD in both forms: the split one at two, fp16, 1024 tokens after 32768 keys
+// 588 -> 678 us, 512 after 16384 174 -> 195, 256 after 4096 the same.)
 template <typename T, bool SPLIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 : 3))) void fa_prefill_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void fa_prefill_kernel(
     const T* __restrict__ q, T* __restrict__ out, const T* __restrict__ kc, const T* __restrict__ vc,
     const int32_t* __restrict__ qseq, const int32_t* __restrict__ qlen, const int32_t* __restrict__ tables,
     int64_t tokens, int q_heads, int kv_heads, int bs, int max_blocks, float scale_log2, int64_t q_stride,
@@ -281,15 +283,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 :
   // registers and padded LDS rows, K ran 614 against 594 us at config 2.)  Keys
   // past the tile's range may hold anything: V's resource ends at the range, so
   // those rows arrive as zeros (their p is 0, and 0 * NaN would not be); K's are
-  // masked in the scores.
-  uint32_t k_off[4], v_off[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = 16 * wave + 4 * i + (lane >> 4);
-    const uint32_t rb = (uint32_t)((int64_t)row * kv_stride * sizeof(T));
-    k_off[i] = rb + 16u * (uint32_t)((lane & 15) ^ (row & 15));
-    v_off[i] = rb + 16u * (uint32_t)((lane & 15) ^ (4 * (row & 3)));
-  }
+  // masked in the scores.  (The rows' part of an offset is uniform between transfers: a lane
+  // keeps its first row's byte and unit, three registers.)
+  const uint32_t row_b = (uint32_t)(kv_stride * sizeof(T));
+  const uint32_t kv_off = (uint32_t)(16 * wave + (lane >> 4)) * row_b;
+  const uint32_t k_unit = (uint32_t)((lane & 15) ^ (lane >> 4)) * 16u;  // row 4 i + lane / 16: ^ 4 i
+  const uint32_t v_off = kv_off + 16u * (uint32_t)((lane & 15) ^ (4 * (lane >> 4)));
   auto chunk_head = [&](int c) {
     const int k0 = c * kFaBk;
     const int64_t row0 = (int64_t)tab[k0 / bs] * bs + k0 % bs;
@@ -301,7 +300,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 :
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rk, (__attribute__((address_space(3))) void*)(dst + (16 * wave + 4 * i) * kFaKRow), 16, k_off[i], 0, 0, 0);
+          rk, (__attribute__((address_space(3))) void*)(dst + (16 * wave + 4 * i) * kFaKRow), 16,
+          kv_off + (k_unit ^ (64u * i)), 4 * i * row_b, 0, 0);
   };
   auto load_v = [&](int c, uint8_t* dst) {
     const int k0 = c * kFaBk;
@@ -311,7 +311,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 :
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rv, (__attribute__((address_space(3))) void*)(dst + (16 * wave + 4 * i) * kFaKRow), 16, v_off[i], 0, 0, 0);
+          rv, (__attribute__((address_space(3))) void*)(dst + (16 * wave + 4 * i) * kFaKRow), 16, v_off,
+          4 * i * row_b, 0, 0);
   };
 
   // The PV operand by transpose reads.  ds_read_b64_tr_b16 over a 16-lane group:
@@ -535,9 +536,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
     int64_t tokens, int q_heads, int kv_heads, int bs, int max_blocks, float scale_log2, int64_t q_stride,
     int64_t tiles, int split_keys, float* __restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int half = lane >> 5;
   const int64_t bid = blockIdx.x;
   const int64_t tile = tiles - 1 - bid / q_heads;  // the longest tiles (latest positions) first
   const int h = (int)(bid % q_heads);
@@ -547,13 +546,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   const int kvh = h / (q_heads / kv_heads);
   const int64_t kv_stride = (int64_t)kv_heads * kFaHd;
   const int tend = tokens - t0 < kFaBq ? (int)(tokens - t0) : kFaBq;
-  // this lane's query (a column of S^T and O^T)
-  const int ql = 32 * wave + (lane & 31);
-  const int64_t tq = t0 + ql;
 
   int r0 = 0;
 #pragma unroll 1
   while (true) {  // the tile's runs [r0, r1)
+  // As fa_prefill_kernel: 224 VGPRs and not 240, with which two workgroups still share a CU but
+  // the last, partial round of them pairs up on fewer CUs (1024 tokens after 32768 keys 4.24 -> 4.86 ms).
+  const int lane = fa_lane();
+  const int half = lane >> 5;
+  // this lane's query (a column of S^T and O^T)
+  const int ql = 32 * wave + (lane & 31);
+  const int64_t tq = t0 + ql;
   const int r1 = runs.end_after(r0, tend);
   const int32_t* tab = tables + (int64_t)qseq[t0 + r0] * max_blocks;
 
@@ -578,7 +581,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
                  : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   // chunk loads: rows ld_r + 8 i (i < 4) of K and V, 16 B column ld_c of each
-  const int tid = threadIdx.x;
+  const int tid = 64 * wave + lane;
   const int ld_c = tid & 31, ld_r = tid >> 5;
   u32x4 kreg[4], vreg[4];
   auto load_chunk = [&](int c) {
@@ -688,27 +691,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   }
 
   // O^T: lane column = query; register j of tile d is dim 4 (8 (j/4) + 4 half + j%4) + d
+  const int lane_e = fa_lane(), half_e = lane_e >> 5, ql_e = 32 * wave + (lane_e & 31);
+  const bool ok_e = ql_e >= r0 && ql_e < r1;
+  const int64_t tq_e = t0 + ql_e;
   if constexpr (SPLIT) {  // unnormalised partial O, running max (exp2 units) and sum
-    if (q_ok) {
-      const int64_t pi = (tq * q_heads + h) * gridDim.z + blockIdx.z;
+    if (ok_e) {
+      const int64_t pi = (tq_e * q_heads + h) * gridDim.z + blockIdx.z;
       float* po = part + pi * kFaHd;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        const int r = 8 * (j >> 2) + 4 * half + (j & 3);
+        const int r = 8 * (j >> 2) + 4 * half_e + (j & 3);
         st16(po + 4 * r, __builtin_bit_cast(u32x4, f32x4{o[0][j], o[1][j], o[2][j], o[3][j]}));
       }
-      if (half == 0) {
+      if (half_e == 0) {
         float* pml = part + tokens * q_heads * gridDim.z * kFaHd + 2 * pi;
         pml[0] = m;
         pml[1] = l;
       }
     }
-  } else if (q_ok) {
+  } else if (ok_e) {
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    float* orow = out + (tq * q_heads + h) * kFaHd;
+    float* orow = out + (tq_e * q_heads + h) * kFaHd;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
-      const int r = 8 * (j >> 2) + 4 * half + (j & 3);
+      const int r = 8 * (j >> 2) + 4 * half_e + (j & 3);
       st16(orow + 4 * r, __builtin_bit_cast(u32x4, f32x4{o[0][j] * inv, o[1][j] * inv, o[2][j] * inv, o[3][j] * inv}));
     }
   }

@@ -3,6 +3,7 @@ rejects bad arguments on the host (no GPU work is issued by these tests)."""
 from __future__ import annotations
 
 import re
+import struct
 import subprocess
 from pathlib import Path
 
@@ -181,3 +182,39 @@ def test_kquant_decode_kernels_opt_into_their_lds_each():
     kernels = [n for n in names if n.startswith("_ZN3nvf14kq_gemv_kernel")]
     flags = [n for n in names if "launch_kv" in n and n.endswith("9attr_once")]
     assert kernels and len(flags) == len(kernels)
+
+
+LLVM = Path("/opt/rocm/llvm/bin")
+
+
+def kernel_vgprs(tmp_path) -> dict[str, int]:
+    """VGPRs of every kernel of the built library, from its code objects' notes."""
+    fat = tmp_path / "fat"
+    subprocess.run([LLVM / "llvm-objcopy", "--dump-section", f".hip_fatbin={fat}", ops.LIB_PATH, tmp_path / "so"], check=True)
+    data, magic, regs = fat.read_bytes(), b"__CLANG_OFFLOAD_BUNDLE__", {}
+    at = data.find(magic)
+    while at >= 0:  # one bundle per source file: [magic][count]{[offset][size][length][target]}
+        pos = at + 32
+        for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):
+            off, size, n = struct.unpack_from("<QQQ", data, pos)
+            if b"gfx950" in data[pos + 24:pos + 24 + n]:
+                (tmp_path / "co").write_bytes(data[at + off:at + off + size])
+                notes = subprocess.run([LLVM / "llvm-readelf", "--notes", tmp_path / "co"], capture_output=True, text=True,
+                                       check=True).stdout
+                for kernel in notes.split("- .agpr_count")[1:]:
+                    regs[re.search(r"\.name:\s+(\S+)", kernel)[1]] = int(re.search(r"\.vgpr_count:\s+(\d+)", kernel)[1])
+            pos += 24 + n
+        at = data.find(magic, at + 24)
+    return regs
+
+
+def test_prefill_attention_registers(tmp_path):
+    """The registers that the prefill attention's workgroups per CU rest on: 168 for three of the
+    16-bit kernel, 224 for two of the fp32 one."""
+    if not (LLVM / "llvm-readelf").exists():
+        pytest.skip("no LLVM tools")
+    regs = kernel_vgprs(tmp_path)
+    fp32 = [v for k, v in regs.items() if "fa_prefill_f32_kernel" in k]
+    f16 = [v for k, v in regs.items() if "fa_prefill_kernel" in k]
+    assert len(f16) == 4 and max(f16) <= 168
+    assert len(fp32) == 2 and max(fp32) <= 224

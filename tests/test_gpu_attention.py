@@ -685,3 +685,28 @@ def test_paged_attention_time_of_decode_tokens_in_a_prompt(gpu, dt):
     t = {name: time(name) for name in args}
     case(f"decode tokens in a prompt dt={dt}: {t}")
     assert t["both"] < 2 * (t["prompt"] + t["decode"])
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=DT_IDS)
+@pytest.mark.parametrize("split", [False, True], ids=["whole", "split"])
+def test_paged_attention_cache_rows_past_the_keys_may_hold_nan(gpu, dt, split):
+    """Rows of a sequence's last block past its keys, and blocks of no sequence, hold NaN: the same bits."""
+    q_heads, kv_heads, hd, bs = 4, 2, 128, 64
+    ctx = [130, 193, 1000, 67, 300, 61, 257]
+    lens = [130, 150, 129, 67, 1, 61, 200]
+    b = H.make_paged(H.rng(77 + dt), ctx, lens, q_heads, kv_heads, hd, bs, dt)
+    used = np.zeros(b.num_blocks * bs, bool)
+    for s, c in enumerate(ctx):
+        j = np.arange(c)
+        used[b.block_tables[s, j // bs] * bs + j % bs] = True
+    nan = {H.F32: np.nan, H.F16: 0x7E00, H.BF16: 0x7FC0}[dt]
+
+    def run(k_cache, v_cache):
+        args = [H.to_dev(b.q, gpu, dt), H.to_dev(k_cache, gpu, dt), H.to_dev(v_cache, gpu, dt),
+                H.to_dev(b.query_seq, gpu), H.to_dev(b.query_key_len, gpu), H.to_dev(b.block_tables, gpu)]
+        return H.to_host(ops.paged_attention(*args, bs, hd ** -0.5, split=split))
+
+    k_nan, v_nan = b.k_cache.copy(), b.v_cache.copy()
+    k_nan[~used], v_nan[~used] = nan, nan
+    case(f"attention NaN rows split={split} dt={dt}")
+    H.assert_bitexact(run(k_nan, v_nan), run(b.k_cache, b.v_cache), "NaN in rows past the keys")
