@@ -244,270 +244,269 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
   int r0 = 0;
 #pragma unroll 1
   while (true) {  // the tile's runs [r0, r1)
-  // The lane is opaque here and again after the chunks, so that what follows from it is
-  // worked out anew rather than kept in registers (168 VGPRs: three workgroups per CU).
-  int lane = fa_lane();
-  const int half = lane >> 5;
-  // this lane's query (a column of S^T and O^T)
-  const int ql = 32 * wave + (lane & 31);
-  const int64_t tq = t0 + ql;
-  const int r1 = runs.end_after(r0, tend);
-  const int32_t* tab = tables + (int64_t)qseq[t0 + r0] * max_blocks;
+    // The lane is opaque here and again after the chunks, so that what follows from it is
+    // worked out anew rather than kept in registers (168 VGPRs: three workgroups per CU).
+    int lane = fa_lane();
+    const int half = lane >> 5;
+    // this lane's query (a column of S^T and O^T)
+    const int ql = 32 * wave + (lane & 31);
+    const int64_t tq = t0 + ql;
+    const int r1 = runs.end_after(r0, tend);
+    const int32_t* tab = tables + (int64_t)qseq[t0 + r0] * max_blocks;
 
-  // the run's longest key range (every wave computes the same value)
-  float lmax = 0.0f;
+    // the run's longest key range (every wave computes the same value)
+    float lmax = 0.0f;
 #pragma unroll
-  for (int i = 0; i < kFaBq / 64; ++i) {
-    const int t = lane + 64 * i;
-    if (t >= r0 && t < r1) lmax = fmaxf(lmax, (float)qlen[t0 + t]);
-  }
-  const int Lmax = (int)wave_max(lmax);
-  const int nchunks = (Lmax + kFaBk - 1) / kFaBk;
+    for (int i = 0; i < kFaBq / 64; ++i) {
+      const int t = lane + 64 * i;
+      if (t >= r0 && t < r1) lmax = fmaxf(lmax, (float)qlen[t0 + t]);
+    }
+    const int Lmax = (int)wave_max(lmax);
+    const int nchunks = (Lmax + kFaBk - 1) / kFaBk;
 
-  const bool q_ok = ql >= r0 && ql < r1;
-  const int L = q_ok ? qlen[tq] : 0;
-  // the smallest key count among the wave's queries (chunks below it need no mask)
-  // (a wave with no query in range takes the masked path; its outputs are not stored)
-  const float lmin = -wave_max(q_ok ? -(float)L : -INFINITY);
-  const int Lmin = lmin < 2.0e9f ? (int)lmin : 0;
-  v8 qf[kFaHd / 16];
+    const bool q_ok = ql >= r0 && ql < r1;
+    const int L = q_ok ? qlen[tq] : 0;
+    // the smallest key count among the wave's queries (chunks below it need no mask)
+    // (a wave with no query in range takes the masked path; its outputs are not stored)
+    const float lmin = -wave_max(q_ok ? -(float)L : -INFINITY);
+    const int Lmin = lmin < 2.0e9f ? (int)lmin : 0;
+    v8 qf[kFaHd / 16];
 #pragma unroll
-  for (int s = 0; s < kFaHd / 16; ++s) {
-    const u32x4 v = q_ok ? ld16(q + tq * q_stride + (int64_t)h * kFaHd + 16 * s + 8 * half) : u32x4{0, 0, 0, 0};
-    qf[s] = __builtin_bit_cast(v8, v);
-  }
+    for (int s = 0; s < kFaHd / 16; ++s) {
+      const u32x4 v = q_ok ? ld16(q + tq * q_stride + (int64_t)h * kFaHd + 16 * s + 8 * half) : u32x4{0, 0, 0, 0};
+      qf[s] = __builtin_bit_cast(v8, v);
+    }
 
-  // K and V by LDS DMA: transfer i of wave w takes key rows 16 w + 4 i + lane / 16
-  // whole, lane l fetching the 16-byte unit that belongs at position l % 16: for K
-  // unit (l % 16) ^ (row % 16), for V unit (l % 16) ^ 4 (row % 4).  (Through
-  // registers and padded LDS rows, K ran 614 against 594 us at config 2.)  Keys
-  // past the tile's range may hold anything: V's resource ends at the range, so
-  // those rows arrive as zeros (their p is 0, and 0 * NaN would not be); K's are
-  // masked in the scores.  (The rows' part of an offset is uniform between transfers: a lane
-  // keeps its first row's byte and unit, three registers.)
-  const uint32_t row_b = (uint32_t)(kv_stride * sizeof(T));
-  const uint32_t kv_off = (uint32_t)(16 * wave + (lane >> 4)) * row_b;
-  const uint32_t k_unit = (uint32_t)((lane & 15) ^ (lane >> 4)) * 16u;  // row 4 i + lane / 16: ^ 4 i
-  const uint32_t v_off = kv_off + 16u * (uint32_t)((lane & 15) ^ (4 * (lane >> 4)));
-  auto chunk_head = [&](int c) {
-    const int k0 = c * kFaBk;
-    const int64_t row0 = (int64_t)tab[k0 / bs] * bs + k0 % bs;
-    return row0 * kv_stride + (int64_t)kvh * kFaHd;
-  };
-  auto load_k = [&](int c, uint8_t* dst) {
-    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<T*>(kc + chunk_head(c)), (short)0, (int)(kFaBk * kv_stride * sizeof(T)), 0x00020000);
+    // K and V by LDS DMA: transfer i of wave w takes key rows 16 w + 4 i + lane / 16
+    // whole, lane l fetching the 16-byte unit that belongs at position l % 16: for K
+    // unit (l % 16) ^ (row % 16), for V unit (l % 16) ^ 4 (row % 4).  (Through
+    // registers and padded LDS rows, K ran 614 against 594 us at config 2.)  Keys
+    // past the tile's range may hold anything: V's resource ends at the range, so
+    // those rows arrive as zeros (their p is 0, and 0 * NaN would not be); K's are
+    // masked in the scores.  (The rows' part of an offset is uniform between transfers: a lane
+    // keeps its first row's byte and unit, three registers.)
+    const uint32_t row_b = (uint32_t)(kv_stride * sizeof(T));
+    const uint32_t kv_off = (uint32_t)(16 * wave + (lane >> 4)) * row_b;
+    const uint32_t k_unit = (uint32_t)((lane & 15) ^ (lane >> 4)) * 16u;  // row 4 i + lane / 16: ^ 4 i
+    const uint32_t v_off = kv_off + 16u * (uint32_t)((lane & 15) ^ (4 * (lane >> 4)));
+    auto chunk_head = [&](int c) {
+      const int k0 = c * kFaBk;
+      const int64_t row0 = (int64_t)tab[k0 / bs] * bs + k0 % bs;
+      return row0 * kv_stride + (int64_t)kvh * kFaHd;
+    };
+    auto load_k = [&](int c, uint8_t* dst) {
+      const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<T*>(kc + chunk_head(c)), (short)0, (int)(kFaBk * kv_stride * sizeof(T)), 0x00020000);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rk, (__attribute__((address_space(3))) void*)(dst + (16 * wave + 4 * i) * kFaKRow), 16,
-          kv_off + (k_unit ^ (64u * i)), 4 * i * row_b, 0, 0);
-  };
-  auto load_v = [&](int c, uint8_t* dst) {
-    const int k0 = c * kFaBk;
-    const int vrows = Lmax - k0 < kFaBk ? Lmax - k0 : kFaBk;
-    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<T*>(vc + chunk_head(c)), (short)0, (int)(vrows * kv_stride * sizeof(T)), 0x00020000);
+      for (int i = 0; i < 4; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rk, (__attribute__((address_space(3))) void*)(dst + (16 * wave + 4 * i) * kFaKRow), 16,
+            kv_off + (k_unit ^ (64u * i)), 4 * i * row_b, 0, 0);
+    };
+    auto load_v = [&](int c, uint8_t* dst) {
+      const int k0 = c * kFaBk;
+      const int vrows = Lmax - k0 < kFaBk ? Lmax - k0 : kFaBk;
+      const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<T*>(vc + chunk_head(c)), (short)0, (int)(vrows * kv_stride * sizeof(T)), 0x00020000);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rv, (__attribute__((address_space(3))) void*)(dst + (16 * wave + 4 * i) * kFaKRow), 16, v_off,
-          4 * i * row_b, 0, 0);
-  };
+      for (int i = 0; i < 4; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rv, (__attribute__((address_space(3))) void*)(dst + (16 * wave + 4 * i) * kFaKRow), 16, v_off,
+            4 * i * row_b, 0, 0);
+    };
 
-  // The PV operand by transpose reads.  ds_read_b64_tr_b16 over a 16-lane group:
-  // lane i receives, as its element e, 16-bit element i % 4 of the 8 bytes that
-  // lane 4 e + i / 4 addresses.  So when lane s of the group addresses key row
-  // key0 + s / 4, dims dim0 + 4 (s % 4) .. + 3, lane i receives dim dim0 + i of
-  // keys key0 .. key0 + 3: the A operand (row = dim, k = key) of the 32x32x16 MFMA.
-  // Lane l: dims 32 d + 16 ((l >> 4) & 1) + 4 (s % 4), keys 4 half + s / 4 (+ 8 for
-  // the operand's second half) past the key step's first, s = l % 16.  Its 16-byte
-  // unit 4 d + 2 ((l >> 4) & 1) + (s % 4) / 2 sits at that ^ 4 (key % 4) = ^ 4 (s / 4):
-  // a lane base per d; the key step and the half are row offsets.  Each 32-lane half
-  // of a read covers 4 keys x 4 units, at 16 distinct positions of one 256-byte row
-  // span: no bank conflicts.
-  uint32_t v_lane[kFaHd / 32];
-  {
-    const int s16 = lane & 15, g16 = (lane >> 4) & 1;
+    // The PV operand by transpose reads.  ds_read_b64_tr_b16 over a 16-lane group:
+    // lane i receives, as its element e, 16-bit element i % 4 of the 8 bytes that
+    // lane 4 e + i / 4 addresses.  So when lane s of the group addresses key row
+    // key0 + s / 4, dims dim0 + 4 (s % 4) .. + 3, lane i receives dim dim0 + i of
+    // keys key0 .. key0 + 3: the A operand (row = dim, k = key) of the 32x32x16 MFMA.
+    // Lane l: dims 32 d + 16 ((l >> 4) & 1) + 4 (s % 4), keys 4 half + s / 4 (+ 8 for
+    // the operand's second half) past the key step's first, s = l % 16.  Its 16-byte
+    // unit 4 d + 2 ((l >> 4) & 1) + (s % 4) / 2 sits at that ^ 4 (key % 4) = ^ 4 (s / 4):
+    // a lane base per d; the key step and the half are row offsets.  Each 32-lane half
+    // of a read covers 4 keys x 4 units, at 16 distinct positions of one 256-byte row
+    // span: no bank conflicts.
+    uint32_t v_lane[kFaHd / 32];
+    {
+      const int s16 = lane & 15, g16 = (lane >> 4) & 1;
 #pragma unroll
-    for (int d = 0; d < kFaHd / 32; ++d)
-      v_lane[d] = (uint32_t)((4 * half + s16 / 4) * kFaKRow + 16 * ((4 * d + 2 * g16 + (s16 & 3) / 2) ^ (4 * (s16 / 4))) +
-                             8 * (s16 & 1));
-  }
+      for (int d = 0; d < kFaHd / 32; ++d)
+        v_lane[d] = (uint32_t)((4 * half + s16 / 4) * kFaKRow +
+                               16 * ((4 * d + 2 * g16 + (s16 & 3) / 2) ^ (4 * (s16 / 4))) + 8 * (s16 & 1));
+    }
 
-  f32x16 o[kFaHd / 32];
+    f32x16 o[kFaHd / 32];
 #pragma unroll
-  for (int d = 0; d < kFaHd / 32; ++d) o[d] = f32x16{};
-  float m = -INFINITY, l = 0.0f;
+    for (int d = 0; d < kFaHd / 32; ++d) o[d] = f32x16{};
+    float m = -INFINITY, l = 0.0f;
 
-  // this workgroup's chunks: all of the run's, or split blockIdx.z's split_keys keys
-  int c0 = 0, c1 = nchunks;
-  if constexpr (SPLIT) {
-    c0 = (int)blockIdx.z * (split_keys / kFaBk);
-    c1 = min(c1, c0 + split_keys / kFaBk);
-  }
-  uint8_t* const vbuf = lds + 2 * kFaKBytes;
-  if (c0 < c1) {
-    load_k(c0, lds);
-    load_v(c0, vbuf);
-  }
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the K transfers are in LDS
-  __syncthreads();
-  for (int c = c0; c < c1; ++c) {
-    const uint8_t* buf = lds + ((c - c0) & 1) * kFaKBytes;
-    // S^T = K . Q^T for keys [32 kt, 32 kt + 32)
-    // (the two key tiles' MFMA chains interleaved: neither waits on its own accumulator)
-    f32x16 st[2] = {f32x16{}, f32x16{}};
-    // Wave priority over the MFMA blocks (S 2 here, PV 1 below), 0 over the softmax: a
-    // SIMD's three waves then hand its issue slots to the one with matrix work first, and
-    // the others' softmax fills the MFMAs' shadow (config 2: 545 -> 536 us with 1 for
-    // both, 555 -> 545 with S above PV on another box; raising the softmax instead: 539).
-    __builtin_amdgcn_s_setprio(2);
+    // this workgroup's chunks: all of the run's, or split blockIdx.z's split_keys keys
+    int c0 = 0, c1 = nchunks;
+    if constexpr (SPLIT) {
+      c0 = (int)blockIdx.z * (split_keys / kFaBk);
+      c1 = min(c1, c0 + split_keys / kFaBk);
+    }
+    uint8_t* const vbuf = lds + 2 * kFaKBytes;
+    if (c0 < c1) {
+      load_k(c0, lds);
+      load_v(c0, vbuf);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the K transfers are in LDS
+    __syncthreads();
+    for (int c = c0; c < c1; ++c) {
+      const uint8_t* buf = lds + ((c - c0) & 1) * kFaKBytes;
+      // S^T = K . Q^T for keys [32 kt, 32 kt + 32)
+      // (the two key tiles' MFMA chains interleaved: neither waits on its own accumulator)
+      f32x16 st[2] = {f32x16{}, f32x16{}};
+      // Wave priority over the MFMA blocks (S 2 here, PV 1 below), 0 over the softmax: a
+      // SIMD's three waves then hand its issue slots to the one with matrix work first, and
+      // the others' softmax fills the MFMAs' shadow (config 2: 545 -> 536 us with 1 for
+      // both, 555 -> 545 with S above PV on another box; raising the softmax instead: 539).
+      __builtin_amdgcn_s_setprio(2);
 #pragma unroll
-    for (int s = 0; s < kFaHd / 16; ++s)
+      for (int s = 0; s < kFaHd / 16; ++s)
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        const int kr = 32 * kt + (lane & 31), ku = 2 * s + half;  // K row, 16-byte unit
-        const v8 a = __builtin_bit_cast(v8, ld16(buf + kr * kFaKRow + 16 * (ku ^ (kr & 15))));
-        st[kt] = M::mma(a, qf[s], st[kt]);
+        for (int kt = 0; kt < 2; ++kt) {
+          const int kr = 32 * kt + (lane & 31), ku = 2 * s + half;  // K row, 16-byte unit
+          const v8 a = __builtin_bit_cast(v8, ld16(buf + kr * kFaKRow + 16 * (ku ^ (kr & 15))));
+          st[kt] = M::mma(a, qf[s], st[kt]);
+        }
+      __builtin_amdgcn_s_setprio(0);
+      if (c + 1 < c1) load_k(c + 1, lds + ((c + 1 - c0) & 1) * kFaKBytes);  // in flight during the softmax and PV
+      // online softmax for this lane's query; element j of tile kt is key
+      // c*64 + 32 kt + 8 (j/4) + 4 half + j%4.  The running max m is kept in
+      // exp2 units (score * scale_log2); since scale_log2 > 0 and rounding is
+      // monotonic, the max of the raw scores times scale_log2 is exactly the max
+      // of the scaled ones, and each p takes one fma into exp2.
+      // (four independent max and sum chains, not one chain of 32 dependent ops)
+      float mx4[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if ((c + 1) * kFaBk <= Lmin) {  // every key of the chunk is visible to every query of the wave
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) mx4[j & 3] = fmaxf(mx4[j & 3], st[kt][j]);
+      } else {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            const int key = c * kFaBk + 32 * kt + 8 * (j >> 2) + 4 * half + (j & 3);
+            const float x = key < L ? st[kt][j] : -INFINITY;
+            st[kt][j] = x;
+            mx4[j & 3] = fmaxf(mx4[j & 3], x);
+          }
       }
-    __builtin_amdgcn_s_setprio(0);
-    if (c + 1 < c1) load_k(c + 1, lds + ((c + 1 - c0) & 1) * kFaKBytes);  // in flight during the softmax and PV
-    // online softmax for this lane's query; element j of tile kt is key
-    // c*64 + 32 kt + 8 (j/4) + 4 half + j%4.  The running max m is kept in
-    // exp2 units (score * scale_log2); since scale_log2 > 0 and rounding is
-    // monotonic, the max of the raw scores times scale_log2 is exactly the max
-    // of the scaled ones, and each p takes one fma into exp2.
-    // (four independent max and sum chains, not one chain of 32 dependent ops)
-    float mx4[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    if ((c + 1) * kFaBk <= Lmin) {  // every key of the chunk is visible to every query of the wave
+      float mx = fmaxf(fmaxf(mx4[0], mx4[1]), fmaxf(mx4[2], mx4[3]));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      // Lazy running max: m moves (and O and l are rescaled) only when some query of the
+      // wave would see a weight above 2^kFaLazy under the current m.  Otherwise the chunk's
+      // weights are taken against the stale m, at most 2^kFaLazy.  O and l always share one
+      // m, so out = O / l is unchanged; only the point where the 16-bit P rounds moves,
+      // with the same relative precision.  With m = -inf (every key so far masked) any
+      // finite candidate moves it.
+      const float m_cand = fmaxf(m, mx * scale_log2);
+      if (__any(m_cand > m + kFaLazy)) {
+        const float alpha = __builtin_amdgcn_exp2f(m - (m_cand == -INFINITY ? 0.0f : m_cand));
+        l *= alpha;
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) mx4[j & 3] = fmaxf(mx4[j & 3], st[kt][j]);
-    } else {
+        for (int d = 0; d < kFaHd / 32; ++d) o[d] *= alpha;
+        m = m_cand;
+      }
+      const float m_use = m == -INFINITY ? 0.0f : m;
+      float ls4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      v8 pb[2][2];
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          const int key = c * kFaBk + 32 * kt + 8 * (j >> 2) + 4 * half + (j & 3);
-          const float x = key < L ? st[kt][j] : -INFINITY;
-          st[kt][j] = x;
-          mx4[j & 3] = fmaxf(mx4[j & 3], x);
+          const float p = __builtin_amdgcn_exp2f(fmaf(st[kt][j], scale_log2, -m_use));
+          ls4[j & 3] += p;
+          pb[kt][j >> 3][j & 7] = (T)p;
         }
-    }
-    float mx = fmaxf(fmaxf(mx4[0], mx4[1]), fmaxf(mx4[2], mx4[3]));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    // Lazy running max: m moves (and O and l are rescaled) only when some query of the
-    // wave would see a weight above 2^kFaLazy under the current m.  Otherwise the chunk's
-    // weights are taken against the stale m, at most 2^kFaLazy.  O and l always share one
-    // m, so out = O / l is unchanged; only the point where the 16-bit P rounds moves,
-    // with the same relative precision.  With m = -inf (every key so far masked) any
-    // finite candidate moves it.
-    const float m_cand = fmaxf(m, mx * scale_log2);
-    if (__any(m_cand > m + kFaLazy)) {
-      const float alpha = __builtin_amdgcn_exp2f(m - (m_cand == -INFINITY ? 0.0f : m_cand));
-      l *= alpha;
-#pragma unroll
-      for (int d = 0; d < kFaHd / 32; ++d) o[d] *= alpha;
-      m = m_cand;
-    }
-    const float m_use = m == -INFINITY ? 0.0f : m;
-    float ls4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    v8 pb[2][2];
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const float p = __builtin_amdgcn_exp2f(fmaf(st[kt][j], scale_log2, -m_use));
-        ls4[j & 3] += p;
-        pb[kt][j >> 3][j & 7] = (T)p;
+      float ls = (ls4[0] + ls4[1]) + (ls4[2] + ls4[3]);
+      ls += __shfl_xor(ls, 32);
+      l += ls;
+      // O^T += V^T . P^T, key step u of tile kt: keys 32 kt + 16 u + 4 half + {0..3, 8..11},
+      // P^T's keys, and V^T's by two transpose reads (+0 and +8 key rows)
+      // V(c): issued after the previous chunk's second barrier, before K(c + 1).  (Bare
+      // barriers: a workgroup fence would add a vmcnt(0) and drain K(c + 1); the
+      // wavefront fences keep the compiler's LDS accesses on their side.)
+      if (c > c0) {
+        if (c + 1 < c1)
+          __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4): all but K(c + 1)
+        else
+          __builtin_amdgcn_s_waitcnt(0x0F70);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
-    float ls = (ls4[0] + ls4[1]) + (ls4[2] + ls4[3]);
-    ls += __shfl_xor(ls, 32);
-    l += ls;
-    // O^T += V^T . P^T, key step u of tile kt: keys 32 kt + 16 u + 4 half + {0..3, 8..11},
-    // P^T's keys, and V^T's by two transpose reads (+0 and +8 key rows)
-    // V(c): issued after the previous chunk's second barrier, before K(c + 1).  (Bare
-    // barriers: a workgroup fence would add a vmcnt(0) and drain K(c + 1); the
-    // wavefront fences keep the compiler's LDS accesses on their side.)
-    if (c > c0) {
-      if (c + 1 < c1)
-        __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4): all but K(c + 1)
-      else
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const uint8_t* vt = vbuf;
+      __builtin_amdgcn_s_setprio(1);
+      // (the four dim tiles' MFMA chains interleaved)
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int d = 0; d < kFaHd / 32; ++d) {
+            typedef short s16x4 __attribute__((ext_vector_type(4)));
+            const uint8_t* r = vt + v_lane[d] + (32 * kt + 16 * u) * kFaKRow;
+            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4*)(r));
+            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4*)(r + 8 * kFaKRow));
+            o[d] = M::mma(__builtin_bit_cast(v8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)), pb[kt][u],
+                          o[d]);
+          }
+      if (c + 1 < c1) {
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): K(c + 1) is in LDS
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_s_barrier();  // and every wave is done with V(c)
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        load_v(c + 1, vbuf);
+      }
     }
-    const uint8_t* vt = vbuf;
-    __builtin_amdgcn_s_setprio(1);
-    // (the four dim tiles' MFMA chains interleaved)
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int d = 0; d < kFaHd / 32; ++d) {
-          typedef short s16x4 __attribute__((ext_vector_type(4)));
-          const uint8_t* r = vt + v_lane[d] + (32 * kt + 16 * u) * kFaKRow;
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) s16x4*)(r));
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) s16x4*)(r + 8 * kFaKRow));
-          o[d] = M::mma(__builtin_bit_cast(v8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)), pb[kt][u],
-                        o[d]);
-        }
-    if (c + 1 < c1) {
-      __builtin_amdgcn_s_setprio(0);
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): K(c + 1) is in LDS
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_s_barrier();  // and every wave is done with V(c)
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      load_v(c + 1, vbuf);
-    }
-  }
 
-  const int lane_e = fa_lane(), half_e = lane_e >> 5, ql_e = 32 * wave + (lane_e & 31);
-  const bool ok_e = ql_e >= r0 && ql_e < r1;
-  const int64_t tq_e = t0 + ql_e;
-  // O^T layout: lane column = query, dims 32 d + 8 (j/4) + 4 half + j%4
-  if constexpr (SPLIT) {  // unnormalised partial O, running max (exp2 units) and sum
-    if (ok_e) {
-      const int64_t pi = (tq_e * q_heads + h) * gridDim.z + blockIdx.z;
-      float* po = part + pi * kFaHd;
+    const int lane_e = fa_lane(), half_e = lane_e >> 5, ql_e = 32 * wave + (lane_e & 31);
+    const bool ok_e = ql_e >= r0 && ql_e < r1;
+    const int64_t tq_e = t0 + ql_e;
+    // O^T layout: lane column = query, dims 32 d + 8 (j/4) + 4 half + j%4
+    if constexpr (SPLIT) {  // unnormalised partial O, running max (exp2 units) and sum
+      if (ok_e) {
+        const int64_t pi = (tq_e * q_heads + h) * gridDim.z + blockIdx.z;
+        float* po = part + pi * kFaHd;
+#pragma unroll
+        for (int d = 0; d < kFaHd / 32; ++d)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            st16(po + 32 * d + 8 * g + 4 * half_e,
+                 __builtin_bit_cast(u32x4, f32x4{o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]}));
+        if (half_e == 0) {
+          float* pml = part + tokens * q_heads * gridDim.z * kFaHd + 2 * pi;
+          pml[0] = m;
+          pml[1] = l;
+        }
+      }
+    } else if (ok_e) {
+      const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+      T* orow = out + (tq_e * q_heads + h) * kFaHd;
 #pragma unroll
       for (int d = 0; d < kFaHd / 32; ++d)
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-          st16(po + 32 * d + 8 * g + 4 * half_e,
-               __builtin_bit_cast(u32x4, f32x4{o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]}));
-      if (half_e == 0) {
-        float* pml = part + tokens * q_heads * gridDim.z * kFaHd + 2 * pi;
-        pml[0] = m;
-        pml[1] = l;
-      }
+        for (int g = 0; g < 4; ++g) {
+          typedef T t4 __attribute__((ext_vector_type(4)));
+          t4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = (T)(o[d][4 * g + e] * inv);
+          *reinterpret_cast<t4*>(orow + 32 * d + 8 * g + 4 * half_e) = v;
+        }
     }
-  } else if (ok_e) {
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    T* orow = out + (tq_e * q_heads + h) * kFaHd;
-#pragma unroll
-    for (int d = 0; d < kFaHd / 32; ++d)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        typedef T t4 __attribute__((ext_vector_type(4)));
-        t4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = (T)(o[d][4 * g + e] * inv);
-        *reinterpret_cast<t4*>(orow + 32 * d + 8 * g + 4 * half_e) = v;
-      }
-  }
-  r0 = r1;
-  if (r0 >= tend) break;
-  __syncthreads();  // the next run's chunks reuse the LDS
+    r0 = r1;
+    if (r0 >= tend) break;
+    __syncthreads();  // the next run's chunks reuse the LDS
   }
 }
-
 
 // ---------------------------------------------------------------------------
 // fp32 caches (the reference's own KV dtype) on the fp32 matrix cores,
@@ -550,180 +549,180 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   int r0 = 0;
 #pragma unroll 1
   while (true) {  // the tile's runs [r0, r1)
-  // As fa_prefill_kernel: 224 VGPRs and not 240, with which two workgroups still share a CU but
-  // the last, partial round of them pairs up on fewer CUs (1024 tokens after 32768 keys 4.24 -> 4.86 ms).
-  const int lane = fa_lane();
-  const int half = lane >> 5;
-  // this lane's query (a column of S^T and O^T)
-  const int ql = 32 * wave + (lane & 31);
-  const int64_t tq = t0 + ql;
-  const int r1 = runs.end_after(r0, tend);
-  const int32_t* tab = tables + (int64_t)qseq[t0 + r0] * max_blocks;
+    // As fa_prefill_kernel: 224 VGPRs and not 240, with which two workgroups still share a CU but
+    // the last, partial round of them pairs up on fewer CUs (1024 tokens after 32768 keys 4.24 -> 4.86 ms).
+    const int lane = fa_lane();
+    const int half = lane >> 5;
+    // this lane's query (a column of S^T and O^T)
+    const int ql = 32 * wave + (lane & 31);
+    const int64_t tq = t0 + ql;
+    const int r1 = runs.end_after(r0, tend);
+    const int32_t* tab = tables + (int64_t)qseq[t0 + r0] * max_blocks;
 
-  float lmax = 0.0f;
+    float lmax = 0.0f;
 #pragma unroll
-  for (int i = 0; i < kFaBq / 64; ++i) {
-    const int t = lane + 64 * i;
-    if (t >= r0 && t < r1) lmax = fmaxf(lmax, (float)qlen[t0 + t]);
-  }
-  const int Lmax = (int)wave_max(lmax);
-  const int nchunks = (Lmax + kF32Bk - 1) / kF32Bk;
-
-  const bool q_ok = ql >= r0 && ql < r1;
-  const int L = q_ok ? qlen[tq] : 0;
-  const float lmin = -wave_max(q_ok ? -(float)L : -INFINITY);
-  const int Lmin = lmin < 2.0e9f ? (int)lmin : 0;
-  // B operand of S^T: this lane's query, dims 64 half + 4 i + e
-  f32x4 qf[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i)
-    qf[i] = q_ok ? __builtin_bit_cast(f32x4, ld16(q + tq * q_stride + (int64_t)h * kFaHd + 64 * half + 4 * i))
-                 : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-  // chunk loads: rows ld_r + 8 i (i < 4) of K and V, 16 B column ld_c of each
-  const int tid = 64 * wave + lane;
-  const int ld_c = tid & 31, ld_r = tid >> 5;
-  u32x4 kreg[4], vreg[4];
-  auto load_chunk = [&](int c) {
-    const int k0 = c * kF32Bk;
-    const int64_t row0 = (int64_t)tab[k0 / bs] * bs + k0 % bs;
-    const float* kb = kc + row0 * kv_stride + (int64_t)kvh * kFaHd + ld_c * 4;
-    const float* vb = vc + row0 * kv_stride + (int64_t)kvh * kFaHd + ld_c * 4;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int key = ld_r + 8 * i;
-      kreg[i] = ld16(kb + (int64_t)key * kv_stride);
-      // keys past the tile's range may hold anything: zero their V (their p is 0).
-      // The row itself lies inside the chunk's block, so the load is unconditional
-      // and only the value is selected (no branch around the load).
-      const u32x4 v = ld16(vb + (int64_t)key * kv_stride);
-      vreg[i] = k0 + key < Lmax ? v : u32x4{0, 0, 0, 0};
+    for (int i = 0; i < kFaBq / 64; ++i) {
+      const int t = lane + 64 * i;
+      if (t >= r0 && t < r1) lmax = fmaxf(lmax, (float)qlen[t0 + t]);
     }
-  };
-  auto store_chunk = [&](uint8_t* st) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      st16(st + (ld_r + 8 * i) * kF32KRow + ld_c * 16, kreg[i]);
-      st16(st + kF32KBytes + (ld_r + 8 * i) * kF32VRow + ld_c * 16, vreg[i]);
-    }
-  };
+    const int Lmax = (int)wave_max(lmax);
+    const int nchunks = (Lmax + kF32Bk - 1) / kF32Bk;
 
-  f32x16 o[4];
+    const bool q_ok = ql >= r0 && ql < r1;
+    const int L = q_ok ? qlen[tq] : 0;
+    const float lmin = -wave_max(q_ok ? -(float)L : -INFINITY);
+    const int Lmin = lmin < 2.0e9f ? (int)lmin : 0;
+    // B operand of S^T: this lane's query, dims 64 half + 4 i + e
+    f32x4 qf[16];
 #pragma unroll
-  for (int d = 0; d < 4; ++d) o[d] = f32x16{};
-  float m = -INFINITY, l = 0.0f;
+    for (int i = 0; i < 16; ++i)
+      qf[i] = q_ok ? __builtin_bit_cast(f32x4, ld16(q + tq * q_stride + (int64_t)h * kFaHd + 64 * half + 4 * i))
+                   : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  // this workgroup's chunks: all of the run's, or split blockIdx.z's split_keys keys
-  int c0 = 0, c1 = nchunks;
-  if constexpr (SPLIT) {
-    c0 = (int)blockIdx.z * (split_keys / kF32Bk);
-    c1 = min(c1, c0 + split_keys / kF32Bk);
-  }
-  if (c0 < c1) {
-    load_chunk(c0);
-    store_chunk(lds);
-  }
-  __syncthreads();
-  for (int c = c0; c < c1; ++c) {
-    const uint8_t* buf = lds + ((c - c0) & 1) * kF32Stage;
-    if (c + 1 < c1) load_chunk(c + 1);  // in flight during this chunk
-    // S^T: lane row (key) lane & 31 of the chunk, dims 64 half + ...
-    f32x16 st = f32x16{};
-    // wave priority as in fa_prefill_kernel: S 2, PV 1, the softmax 0 (3957-3968 ->
-    // 3900-3908 us at config 2)
-    __builtin_amdgcn_s_setprio(2);
-    const uint8_t* krow = buf + (lane & 31) * kF32KRow + 256 * half;
+    // chunk loads: rows ld_r + 8 i (i < 4) of K and V, 16 B column ld_c of each
+    const int tid = 64 * wave + lane;
+    const int ld_c = tid & 31, ld_r = tid >> 5;
+    u32x4 kreg[4], vreg[4];
+    auto load_chunk = [&](int c) {
+      const int k0 = c * kF32Bk;
+      const int64_t row0 = (int64_t)tab[k0 / bs] * bs + k0 % bs;
+      const float* kb = kc + row0 * kv_stride + (int64_t)kvh * kFaHd + ld_c * 4;
+      const float* vb = vc + row0 * kv_stride + (int64_t)kvh * kFaHd + ld_c * 4;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const f32x4 a = __builtin_bit_cast(f32x4, ld16(krow + 16 * i));
+      for (int i = 0; i < 4; ++i) {
+        const int key = ld_r + 8 * i;
+        kreg[i] = ld16(kb + (int64_t)key * kv_stride);
+        // keys past the tile's range may hold anything: zero their V (their p is 0).
+        // The row itself lies inside the chunk's block, so the load is unconditional
+        // and only the value is selected (no branch around the load).
+        const u32x4 v = ld16(vb + (int64_t)key * kv_stride);
+        vreg[i] = k0 + key < Lmax ? v : u32x4{0, 0, 0, 0};
+      }
+    };
+    auto store_chunk = [&](uint8_t* st) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) st = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], qf[i][e], st, 0, 0, 0);
+      for (int i = 0; i < 4; ++i) {
+        st16(st + (ld_r + 8 * i) * kF32KRow + ld_c * 16, kreg[i]);
+        st16(st + kF32KBytes + (ld_r + 8 * i) * kF32VRow + ld_c * 16, vreg[i]);
+      }
+    };
+
+    f32x16 o[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) o[d] = f32x16{};
+    float m = -INFINITY, l = 0.0f;
+
+    // this workgroup's chunks: all of the run's, or split blockIdx.z's split_keys keys
+    int c0 = 0, c1 = nchunks;
+    if constexpr (SPLIT) {
+      c0 = (int)blockIdx.z * (split_keys / kF32Bk);
+      c1 = min(c1, c0 + split_keys / kF32Bk);
     }
-    __builtin_amdgcn_s_setprio(0);
-    // online softmax for this lane's query over its keys c*32 + 8 (j/4) + 4 half + j%4
-    // (the running max in exp2 units, as in fa_prefill_kernel)
-    float mx = -INFINITY;
-    if ((c + 1) * kF32Bk <= Lmin) {
+    if (c0 < c1) {
+      load_chunk(c0);
+      store_chunk(lds);
+    }
+    __syncthreads();
+    for (int c = c0; c < c1; ++c) {
+      const uint8_t* buf = lds + ((c - c0) & 1) * kF32Stage;
+      if (c + 1 < c1) load_chunk(c + 1);  // in flight during this chunk
+      // S^T: lane row (key) lane & 31 of the chunk, dims 64 half + ...
+      f32x16 st = f32x16{};
+      // wave priority as in fa_prefill_kernel: S 2, PV 1, the softmax 0 (3957-3968 ->
+      // 3900-3908 us at config 2)
+      __builtin_amdgcn_s_setprio(2);
+      const uint8_t* krow = buf + (lane & 31) * kF32KRow + 256 * half;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) mx = fmaxf(mx, st[j]);
-    } else {
+      for (int i = 0; i < 16; ++i) {
+        const f32x4 a = __builtin_bit_cast(f32x4, ld16(krow + 16 * i));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], qf[i][e], st, 0, 0, 0);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      // online softmax for this lane's query over its keys c*32 + 8 (j/4) + 4 half + j%4
+      // (the running max in exp2 units, as in fa_prefill_kernel)
+      float mx = -INFINITY;
+      if ((c + 1) * kF32Bk <= Lmin) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) mx = fmaxf(mx, st[j]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const int key = c * kF32Bk + 8 * (j >> 2) + 4 * half + (j & 3);
+          const float x = key < L ? st[j] : -INFINITY;
+          st[j] = x;
+          mx = fmaxf(mx, x);
+        }
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      // lazy running max, as in fa_prefill_kernel (P stays fp32 here: no rounding moves)
+      const float m_cand = fmaxf(m, mx * scale_log2);
+      if (__any(m_cand > m + kFaLazy)) {
+        const float alpha = __builtin_amdgcn_exp2f(m - (m_cand == -INFINITY ? 0.0f : m_cand));
+        l *= alpha;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) o[d] *= alpha;
+        m = m_cand;
+      }
+      const float m_use = m == -INFINITY ? 0.0f : m;
+      float ls = 0.0f;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        const int key = c * kF32Bk + 8 * (j >> 2) + 4 * half + (j & 3);
-        const float x = key < L ? st[j] : -INFINITY;
-        st[j] = x;
-        mx = fmaxf(mx, x);
+        st[j] = __builtin_amdgcn_exp2f(fmaf(st[j], scale_log2, -m_use));
+        ls += st[j];
       }
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    // lazy running max, as in fa_prefill_kernel (P stays fp32 here: no rounding moves)
-    const float m_cand = fmaxf(m, mx * scale_log2);
-    if (__any(m_cand > m + kFaLazy)) {
-      const float alpha = __builtin_amdgcn_exp2f(m - (m_cand == -INFINITY ? 0.0f : m_cand));
-      l *= alpha;
+      ls += __shfl_xor(ls, 32);
+      l += ls;
+      // O^T += V^T . P^T: MFMA s takes key 8 (s/4) + 4 half + s%4 (P^T = st[s]); lane
+      // row r = lane & 31 of tile d is dim 4 r + d
+      const uint8_t* vrow = buf + kF32KBytes + 16 * (lane & 31);
+      __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int d = 0; d < 4; ++d) o[d] *= alpha;
-      m = m_cand;
-    }
-    const float m_use = m == -INFINITY ? 0.0f : m;
-    float ls = 0.0f;
+      for (int s = 0; s < 16; ++s) {
+        const int key = 8 * (s >> 2) + 4 * half + (s & 3);
+        const f32x4 a = __builtin_bit_cast(f32x4, ld16(vrow + key * kF32VRow));
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      st[j] = __builtin_amdgcn_exp2f(fmaf(st[j], scale_log2, -m_use));
-      ls += st[j];
+        for (int d = 0; d < 4; ++d) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d], st[s], o[d], 0, 0, 0);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      if (c + 1 < c1) store_chunk(lds + ((c + 1 - c0) & 1) * kF32Stage);
+      __syncthreads();
     }
-    ls += __shfl_xor(ls, 32);
-    l += ls;
-    // O^T += V^T . P^T: MFMA s takes key 8 (s/4) + 4 half + s%4 (P^T = st[s]); lane
-    // row r = lane & 31 of tile d is dim 4 r + d
-    const uint8_t* vrow = buf + kF32KBytes + 16 * (lane & 31);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      const int key = 8 * (s >> 2) + 4 * half + (s & 3);
-      const f32x4 a = __builtin_bit_cast(f32x4, ld16(vrow + key * kF32VRow));
-#pragma unroll
-      for (int d = 0; d < 4; ++d) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d], st[s], o[d], 0, 0, 0);
-    }
-    __builtin_amdgcn_s_setprio(0);
-    if (c + 1 < c1) store_chunk(lds + ((c + 1 - c0) & 1) * kF32Stage);
-    __syncthreads();
-  }
 
-  // O^T: lane column = query; register j of tile d is dim 4 (8 (j/4) + 4 half + j%4) + d
-  const int lane_e = fa_lane(), half_e = lane_e >> 5, ql_e = 32 * wave + (lane_e & 31);
-  const bool ok_e = ql_e >= r0 && ql_e < r1;
-  const int64_t tq_e = t0 + ql_e;
-  if constexpr (SPLIT) {  // unnormalised partial O, running max (exp2 units) and sum
-    if (ok_e) {
-      const int64_t pi = (tq_e * q_heads + h) * gridDim.z + blockIdx.z;
-      float* po = part + pi * kFaHd;
+    // O^T: lane column = query; register j of tile d is dim 4 (8 (j/4) + 4 half + j%4) + d
+    const int lane_e = fa_lane(), half_e = lane_e >> 5, ql_e = 32 * wave + (lane_e & 31);
+    const bool ok_e = ql_e >= r0 && ql_e < r1;
+    const int64_t tq_e = t0 + ql_e;
+    if constexpr (SPLIT) {  // unnormalised partial O, running max (exp2 units) and sum
+      if (ok_e) {
+        const int64_t pi = (tq_e * q_heads + h) * gridDim.z + blockIdx.z;
+        float* po = part + pi * kFaHd;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const int r = 8 * (j >> 2) + 4 * half_e + (j & 3);
+          st16(po + 4 * r, __builtin_bit_cast(u32x4, f32x4{o[0][j], o[1][j], o[2][j], o[3][j]}));
+        }
+        if (half_e == 0) {
+          float* pml = part + tokens * q_heads * gridDim.z * kFaHd + 2 * pi;
+          pml[0] = m;
+          pml[1] = l;
+        }
+      }
+    } else if (ok_e) {
+      const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+      float* orow = out + (tq_e * q_heads + h) * kFaHd;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int r = 8 * (j >> 2) + 4 * half_e + (j & 3);
-        st16(po + 4 * r, __builtin_bit_cast(u32x4, f32x4{o[0][j], o[1][j], o[2][j], o[3][j]}));
-      }
-      if (half_e == 0) {
-        float* pml = part + tokens * q_heads * gridDim.z * kFaHd + 2 * pi;
-        pml[0] = m;
-        pml[1] = l;
+        st16(orow + 4 * r,
+             __builtin_bit_cast(u32x4, f32x4{o[0][j] * inv, o[1][j] * inv, o[2][j] * inv, o[3][j] * inv}));
       }
     }
-  } else if (ok_e) {
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    float* orow = out + (tq_e * q_heads + h) * kFaHd;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int r = 8 * (j >> 2) + 4 * half_e + (j & 3);
-      st16(orow + 4 * r, __builtin_bit_cast(u32x4, f32x4{o[0][j] * inv, o[1][j] * inv, o[2][j] * inv, o[3][j] * inv}));
-    }
-  }
-  r0 = r1;
-  if (r0 >= tend) break;
-  __syncthreads();  // the next run's chunks reuse the LDS
+    r0 = r1;
+    if (r0 >= tend) break;
+    __syncthreads();  // the next run's chunks reuse the LDS
   }
 }
-
 
 // ---------------------------------------------------------------------------
 // The decode kernels' end: a workgroup is one (token, kv head) whose 4 waves each
