@@ -591,15 +591,52 @@ int launch_kq_tile(const void* x, const uint8_t* w, void* out, int64_t m, int64_
   return launch_status("dense_gemm (K-quant)");
 }
 
+// The tile: the one whose estimated time per superblock of the whole output is least, from the
+// tiles that the fullest of the 256 CUs gets (c).  One takes `alone`; where the LDS lets several
+// share a CU each further one adds `busy`, else c of them take `busy` each.  us per superblock
+// (launch time at k = 3584 over 14; 32-, 64-, 128-, 256-row tiles):
+//                      alone                     busy                        from
+//   fp16 Q4_K, Q5_K    2.75 3.25 3.86 5.00       1.3  2.0  3.86 5.35         16 to 4096 x 3584, 4608, 37888 x 3584
+//   bf16 Q4_K, Q5_K    4.25 5.00 6.25 7.80       4.1  5.0  6.25 8.00         32 to 2048 x 4608, 37888 x 3584
+//   Q6_K               4.70 5.40 7.00 6.85       3.55 6.2  7.50 7.20         as the first, and 3584 x 18944
+// (Q6_K is never best at 128 rows: not built.)
+// So 128 rows on 4608 columns take 39 us at 32 rows per tile against 46 to 70 at the others, 1021 rows
+// there 77 at 256 against 102 to 110, 64 x 37888 62 at 64 rows; Q6_K, 1021 x 4608, 107 at 256
+// against 210 to 261.  At each of these sizes the choice is the best tile or within 3% of it.
+template <typename T, int KIND>
+int kq_tile(int64_t m, int64_t n) {
+  constexpr int kCls = KIND == NVF_Q6_K ? 2 : __is_same(T, _Float16) ? 0 : 1;
+  constexpr double kAlone[3][4] = {{2.75, 3.25, 3.86, 5.0}, {4.25, 5.0, 6.25, 7.8}, {4.7, 5.4, 7.0, 6.85}};
+  constexpr double kBusy[3][4] = {{1.3, 2.0, 3.86, 5.35}, {4.1, 5.0, 6.25, 8.0}, {3.55, 6.2, 7.5, 7.2}};
+  int best = 3;
+  double best_t = 0.0;
+  for (int i = 3; i >= 0; --i) {
+    const int64_t bm = 32ll << i, tiles = ((m + bm - 1) / bm) * ((n + kKqBN - 1) / kKqBN);
+    if ((i < 3 && tiles > INT32_MAX) || (i == 2 && KIND == NVF_Q6_K)) continue;
+    const double c = (double)((tiles + 255) / 256);
+    const bool share = i == 0 || (i == 1 && kCls == 0);
+    const double t = c == 1.0 ? kAlone[kCls][i] : share ? kAlone[kCls][i] + (c - 1.0) * kBusy[kCls][i] : c * kBusy[kCls][i];
+    if (i == 3 || t < best_t) {
+      best = i;
+      best_t = t;
+    }
+  }
+  return best;
+}
+
 template <typename T, int KIND, int LAYOUT, typename TO>
 int launch_kq(const void* x, const uint8_t* w, void* out, int64_t m, int64_t n, int64_t k, hipStream_t st) {
-  const int64_t tiles_n = (n + kKqBN - 1) / kKqBN;
-  if (m > 128 && ((m + 255) / 256) * tiles_n >= 192)
-    return launch_kq_tile<T, KIND, LAYOUT, TO, 256, 4, 2>(x, w, out, m, n, k, st);
-  if (m > 64 && ((m + 127) / 128) * tiles_n >= 192)
-    return launch_kq_tile<T, KIND, LAYOUT, TO, 128, 2, 2>(x, w, out, m, n, k, st);
-  if (m > 32) return launch_kq_tile<T, KIND, LAYOUT, TO, 64, 2, 2>(x, w, out, m, n, k, st);
-  return launch_kq_tile<T, KIND, LAYOUT, TO, 32, 1, 4>(x, w, out, m, n, k, st);
+  switch (kq_tile<T, KIND>(m, n)) {
+    case 3:
+      return launch_kq_tile<T, KIND, LAYOUT, TO, 256, 4, 2>(x, w, out, m, n, k, st);
+    case 2:
+      return launch_kq_tile<T, KIND, LAYOUT, TO, KIND == NVF_Q6_K ? 256 : 128, KIND == NVF_Q6_K ? 4 : 2, 2>(x, w, out, m,
+                                                                                                          n, k, st);
+    case 1:
+      return launch_kq_tile<T, KIND, LAYOUT, TO, 64, 2, 2>(x, w, out, m, n, k, st);
+    default:
+      return launch_kq_tile<T, KIND, LAYOUT, TO, 32, 1, 4>(x, w, out, m, n, k, st);
+  }
 }
 
 template <typename T, typename TO>

@@ -94,8 +94,9 @@ KQ_SIZES = [
     (13, 16400, 2304),   # x in several stages, all four results per lane
     (2, 40, 8192),       # narrow and deep
     (17, 130, 256),      # 32: one superblock, two columns in the last tile
-    (33, 129, 2304),     # 64
-    (65, 24577, 256),    # 128
+    (33, 129, 2304),     # 32, a second row of tiles
+    (300, 3500, 256),    # 64
+    (65, 24577, 256),    # 128 (Q6_K: 256)
     (129, 24580, 512),   # 256, one row in the last tile
 ]
 
