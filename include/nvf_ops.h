@@ -262,8 +262,8 @@ int64_t nvf_moe_ffn_workspace_size(int64_t rows, int64_t H, int64_t I, int64_t K
 /* MoE expert FFN (replaces hip_moe_ffn, hip_ops.hpp:38-40): x [rows, H] in x_dtype, out
  * [rows, H] in out_dtype (out += ...), expert weights fp16 (w_bf16 0) or bf16, expert slots
  * in [0, slots) (slots <= 65536; other pairs and pairs with score 0 are skipped).  The pairs
- * are grouped by slot and run as matrix products on the fp32 matrix cores; the k results of
- * a token are summed in k order.  `work`: 16-byte aligned, nvf_moe_ffn_workspace_size bytes. */
+ * are grouped by slot and run as matrix products, exact in fp32 (bf16 experts: activations as
+ * exact bf16 pieces on the bf16 matrix cores); the k results of a token are summed in k order.  `work`: 16-byte aligned, nvf_moe_ffn_workspace_size bytes. */
 int nvf_moe_ffn_ws(const void* x, int x_dtype, const int32_t* idx, const float* score, const void* gu,
                    const void* dn, int w_bf16, const int32_t* slot_of, int64_t rows, int64_t H, int64_t I, int64_t K,
                    int64_t slots, void* out, int out_dtype, void* work, int64_t work_bytes, void* stream);

@@ -29,7 +29,7 @@ int launch_tile16(const void* x, const void* w, void* out, int64_t m, int64_t n,
 // (the latency of its load, wait and barrier); beyond, tiles whose LDS lets two share a
 // CU add `busy` for each further tile per CU, and the others run in whole rounds of
 // `busy`.  Measured in us per step at bf16 (launch time / K steps), on:
-//   256 x 256      alone 1.60 (300 x 24576 x 4096)   round 1.74 (4096 x 24576 x 4096: 669 us, 1232 TFLOP/s)
+//   256 x 256      alone 1.60 (300 x 24576 x 4096)   round 1.74 (4096 x 24576 x 4096: 669 us on that box)
 //   128 x 128      0.64 (1021 x 3584 x 18944)        + 0.60 (1021 x 37888 x 3584: 345 us)
 //   the same, 2 K groups   0.55 (1021 x 3584 x 18944: 163 us against 190)
 //   64 x 128       0.41 (200 x 3584 x 18944)         + 0.35 (4096 x 24576 x 4096: 1080 us)

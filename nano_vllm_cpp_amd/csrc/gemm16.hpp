@@ -7,8 +7,8 @@
 // per stage.  A wave of the 256 x 256 tile owns 128 x 64 outputs: 6 KB of LDS reads per 8
 // MFMAs, three quarters of the LDS rate that a 64 x 64 wave would need.  4096 x 24576 x
 // 4096 bf16: 2298 us on the three-piece split tile kernel (which takes any activation
-// type) -> 669 us, 1232 TFLOP/s; other shapes of the tile and of the stages on the same
-// product: 4 stages of 32 K-values 697 us, 4 waves of 128 x 128 755, 256 x 128 760.
+// type) -> 690 us, 1195 TFLOP/s (670 to 725 over boxes); other shapes of the tile and of the
+// stages, where this one took 669: 4 stages of 32 K-values 697 us, 4 waves of 128 x 128 755, 256 x 128 760.
 // 24 x 151936 x 4096 (LM head): 447 -> 215 us, 5.8 TB/s of weights.
 #pragma once
 

@@ -27,7 +27,7 @@
 // where the plain product has an infinity or a number.  Any of them leaves the output
 // non-finite, and such outputs are made again from the decoded weights on the fp32 matrix
 // cores, by the waves that hold them (1021 x 4096 x 3584, every activation NaN: 13.8 ms one
-// output after the other, 572 us so, 315 on the fp32 tile kernel).
+// output after the other, 520 us so, 315 on the fp32 tile kernel).
 
 #include <array>
 #include <mutex>

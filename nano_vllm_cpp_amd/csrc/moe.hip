@@ -765,7 +765,10 @@ __global__ __launch_bounds__(WM* WN* KG * 64) __attribute__((amdgpu_waves_per_eu
 
 // How a call runs.  Grouping: one workgroup counting in LDS, up to kGroupSlots slots and
 // kGroupPairs pairs (256 rows x top 8: 19 us in four launches -> 5.8); else the one-launch
-// sort, up to 4096 pairs (the drop-in, which does not know its slots); else four launches.
+// sort, up to 4096 pairs (the drop-in, which does not know its slots); else four launches.  A
+// whole call on small experts (H 256, I 64), grouped so / by the others, us: 128 slots, 512
+// pairs 18.9 / 26.8, 4096 29 / 88, 8192 40 / 48, 16384 62 / 70; 16 slots, 16384 pairs 59 / 119;
+// 4096 slots, 2048 pairs 68 / 89, 8192 146 / 144, 16384 274 / 259.
 // Products with bf16 weights: moe16_kernel over tiles of 32, 64 or 128 rows by the pairs per
 // expert that a call brings; the FFN of Qwen3-30B-A3B's experts on bf16 x, us, from the
 // products below: 2 rows 51 -> 43, 16 rows 204 -> 182, 256 rows 389 -> 268, 1024 rows 590 -> 406,
