@@ -342,20 +342,20 @@ int launch_dense(const void* x, const Src& src, void* out, int64_t m, int64_t n,
 // Where the 16-bit matrix-core decode product of kq_gemv.hip beats the products on decoded
 // weights above.  Q4_K, us (there / here), weights not in the cache:
 //   fp16 x, m =                1            2            4            8            16
-//   151936 x 4096        82 / 136     80 / 153     86 / 247    101 / 249    130 / 253
-//   37888 x 3584       22.8 / 26.4  24.3 / 33.4  25.2 / 55.0  29.2 / 56.1  37.8 / 58.1
-//   4608 x 3584             / 9.9        / 9.8   12.0 / 14.6  15.7 / 14.7       / 15.5
-//   3584 x 18944       17.4 / 17.1  19.6 / 22.9  25.0 / 38.6  35.1 / 38.8       / 38.8
+//   151936 x 4096        80 / 136     79 / 153     84 / 247    101 / 249    130 / 253
+//   37888 x 3584       22.5 / 26.4  23.5 / 33.4  24.4 / 55.0  29.3 / 56.1  38.0 / 58.1
+//   4608 x 3584             / 9.9        / 9.8   11.7 / 14.6  15.7 / 14.7       / 15.5
+//   3584 x 18944       17.4 / 17.1  19.1 / 22.9  23.8 / 38.6  35.2 / 38.8       / 38.8
 //   bf16 x
-//   151936 x 4096        91 / 132     95 / 153    101 / 246    117 / 248    147 / 252
-//   37888 x 3584       29.8 / 27.2  30.4 / 38.9  31.4 / 54.5  35.5 / 55.2  43.5 / 56.8
-//   4608 x 3584             / 9.9        / 9.8   13.1 / 14.1  16.4 / 14.3       / 15.3
-//   3584 x 18944            / 17.2  23.3 / 23.1  27.8 / 38.3  37.9 / 38.3       / 38.5
+//   151936 x 4096        88 / 132     91 / 153     98 / 246    117 / 248    147 / 252
+//   37888 x 3584       29.8 / 27.2  29.3 / 38.9  29.7 / 54.5  35.4 / 55.2  43.8 / 56.8
+//   4608 x 3584             / 9.9        / 9.8   12.9 / 14.1  16.4 / 14.3       / 15.3
+//   3584 x 18944            / 17.2  23.3 / 23.1  26.5 / 38.3  38.0 / 38.3       / 38.5
 //   fp32 x
-//   151936 x 4096       112 / 153    115 / 194    126 / 247    150 / 252    227 / 266
-//   37888 x 3584       34.4 / 32.0  34.7 / 45.5  37.9 / 54.5  44.7 / 57.0  70.8 / 70.3
-//   3584 x 18944            / 22.5  27.3 / 33.8  34.3 / 35.4       / 35.4       / 44.0
-// (Q5_K, one row, 37888 x 3584: fp16 29.1 / 39.4, bf16 34.9 / 39.2, fp32 39.4 / 46.1.)  Narrow
+//   151936 x 4096       109 / 153    113 / 194    124 / 247    152 / 252    227 / 266
+//   37888 x 3584       34.4 / 32.0  33.6 / 45.5  37.1 / 54.5  44.8 / 57.0  71.0 / 70.3
+//   3584 x 18944            / 22.5  26.2 / 33.8  33.0 / 35.4       / 35.4       / 44.0
+// (Q5_K, one row, 37888 x 3584: fp16 28.7 / 39.4, bf16 34.8 / 39.2, fp32 39.0 / 46.1.)  Narrow
 // outputs have few workgroups over which to spread its staging of x.
 bool kq_gemv_wins(int w_format, int x_dtype, int64_t m, int64_t n, int64_t k) {
   const bool f16 = x_dtype == NVF_F16, deep = k >= 8192;

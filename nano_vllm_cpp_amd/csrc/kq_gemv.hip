@@ -9,8 +9,8 @@
 // sc_j (q - c_j) 2^-14, so v_mfma_f32_16x16x32 sums whole superblocks for 16 rows and 16 columns,
 // and d takes one fused multiply-add per four rows and 4096 weights.  bf16 x (and fp32 x as
 // three exact bf16 pieces): the operand is q - c_j, and sc_j takes one multiply-add per four rows
-// and 512 weights.  The r_j are two MFMAs per superblock, over the sub-blocks' sums of x (both
-// as three bf16 pieces).  The result is within three times the bound of fp32 sums of x w.
+// and 512 weights.  The r_j times the sub-blocks' sums of x are 8 multiply-adds per superblock up to
+// 4 rows, else two MFMAs (both as three bf16 pieces).  The result is within three times the bound of fp32 sums of x w.
 //
 // A wave owns 16 columns: lane l holds column l % 16 and, of every sub-block, the values
 // 8 (l / 16) .. + 7.  Read straight from memory in that layout a superblock takes 5 loads that
@@ -20,12 +20,13 @@
 // workgroup on other columns share the staged x; KG groups of them split K for
 // narrow outputs.
 //
-// fp16 x, Q4_K: 1 x 151936 x 4096 (350 MB) 136 us on decoded weights -> 82 (4.3 TB/s); 1 x
-// 37888 x 3584 26.4 -> 22.8 us, 8 x 37888 x 3584 56 -> 29.2.  160 VALU instructions per
-// superblock of a wave's 16 columns, 2.5 per weight; with c_j = 0 (no centres: the bound then lies over the two parts, however
-// they cancel) the three take 73, 21.0 and 26.5 us; with a subtraction of c_j and a
-// multiply-add per sub-block 85, 23.6 and 30.5.  bf16 x, 2 x 37888 x 3584: 30.4 us, 34.6 with the
-// subtraction in fp32 after the conversion.
+// fp16 x, Q4_K: 1 x 151936 x 4096 (350 MB) 136 us on decoded weights -> 80 (4.4 TB/s); 1 x
+// 37888 x 3584 26.4 -> 22.5 us, 8 x 37888 x 3584 56 -> 29.3.  146 VALU instructions per
+// superblock of a wave's 16 columns (2.3 per weight); with the remainders by MFMAs at one row too
+// 160 and 22.8 us; with a subtraction of c_j and a multiply-add per sub-block 174 and 23.6; with
+// c_j = 0 (no centres: the bound then lies over the two parts, however they cancel) the three
+// take 73, 21.0 and 26.5 us.  bf16 x, 2 x 37888 x 3584: 29.3 us, 34.6 with the subtraction in
+// fp32 after the conversion.
 //
 // Infinities and NaN: sums that come out non-finite are made again from the decoded weights,
 // as in kq_gemm.hip (8 x 37888 x 3584, every activation NaN: 1040 us one
@@ -190,7 +191,8 @@ __device__ __forceinline__ void kv_gather(uint32_t v, uint32_t* o) {
 
 // x as staged: XP planes of 16-bit values (fp32: three exact bf16 pieces), rows of a
 // superblock 528 bytes apart (the 16 rows of a read phase on distinct banks), then the
-// sub-blocks' sums' bf16 pieces, [row][8 j][x0 x0 x0 x1 x1 x2 0 0], rows 144 bytes apart.
+// sub-blocks' sums: as bf16 pieces, [row][8 j][x0 x0 x0 x1 x1 x2 0 0], rows 144 bytes apart, or
+// up to 4 rows as they are, [8 j][4 rows].
 template <typename TX>
 struct KvX {
   using T = TX;
@@ -204,7 +206,7 @@ struct KvX<float> {
 constexpr int kKvRow = 528, kKvSums = 144;
 template <typename TX>
 constexpr int kv_sb_bytes(int m) {
-  return m * (KvX<TX>::kPlanes * kKvRow + kKvSums);
+  return m * KvX<TX>::kPlanes * kKvRow + (m <= 4 ? 128 : m * kKvSums);
 }
 
 // A weight stage in LDS: one superblock of 16 columns, column after column.  A column is 9 or
@@ -289,10 +291,15 @@ __global__ __launch_bounds__(WC* KG * 64) __attribute__((amdgpu_waves_per_eu(2, 
       for (int e = 0; e < 8; ++e) sum += v[e];
       sum = group_sum<4>(sum);
       if ((ch & 3) == 0) {
-        uint32_t pc[3];
-        bf16_pieces(sum, pc);
-        st16(xl + s * sbb + XP * m * kKvRow + r * kKvSums + 4 * ch,
-             u32x4{pc[0] | pc[0] << 16, pc[0] | pc[1] << 16, pc[1] | pc[2] << 16, 0u});
+        uint8_t* ds = xl + s * sbb + XP * m * kKvRow;
+        if constexpr (NE == 1) {
+          reinterpret_cast<float*>(ds)[ch + r] = sum;
+        } else {
+          uint32_t pc[3];
+          bf16_pieces(sum, pc);
+          st16(ds + r * kKvSums + 4 * ch,
+               u32x4{pc[0] | pc[0] << 16, pc[0] | pc[1] << 16, pc[1] | pc[2] << 16, 0u});
+        }
       }
     }
   };
@@ -303,14 +310,16 @@ __global__ __launch_bounds__(WC* KG * 64) __attribute__((amdgpu_waves_per_eu(2, 
   f32x4 tot = {};
   const int xr = (c >> 2) + 4 * (c & 3), xrow = xr < m ? xr : 0;
   const uint8_t* const xa = xl + xrow * kKvRow + 16 * g;
-  const uint8_t* const xs = xl + XP * m * kKvRow + xrow * kKvSums + 32 * g;
+  const uint8_t* const xs = xl + XP * m * kKvRow + (NE == 1 ? 0 : xrow * kKvSums) + 32 * g;
+  float rt[4] = {};  // NE = 1: the remainders' part of rows 0 .. 3, of this lane group's sub-blocks
   auto compute = [&](const Raw& r, int s) {  // superblock s of the staged chunk
     const uint8_t* xb = xa + s * sbb;
     const float d = r.d();
     uint32_t sc[2], mn[2];
     q4k_tables(r.hdr, sc, mn);
-    // lane group g finds the centres of sub-blocks 2 g and 2 g + 1 and holds their remainders
-    // as [r0 r1 r2 r0 r1 r0 0 0]
+    // lane group g finds the centres of sub-blocks 2 g and 2 g + 1 and takes their remainders: up to
+    // 4 rows times the sums of x as they are (8 multiply-adds), else by an MFMA over the pieces
+    // [r0 r1 r2 r0 r1 r0 0 0]
     const uint32_t sg = (g < 2 ? sc[0] : sc[1]) >> (16 * (g & 1)), mg = (g < 2 ? mn[0] : mn[1]) >> (16 * (g & 1));
     uint32_t sub[2][4];
 #pragma unroll
@@ -318,10 +327,18 @@ __global__ __launch_bounds__(WC* KG * 64) __attribute__((amdgpu_waves_per_eu(2, 
       const float sf = (float)byte_of(sg, i), p = d * sf, o = r.dmin() * (float)byte_of(mg, i);
       const float q0 = kq_centre(p, o, Raw::kTop);
       kv_gather(kv_sub<Raw>(sf, q0, i == 1, T{}), sub[i]);
-      uint32_t pc[3];
-      bf16_pieces(fmaf(p, q0, -o), pc);
-      const u32x4 rb = {pc[0] | pc[1] << 16, pc[2] | pc[0] << 16, pc[1] | pc[0] << 16, 0u};
-      tot = mfma16x16(ld16(xs + s * sbb + 16 * i), rb, tot, __bf16{});
+      const float rem = fmaf(p, q0, -o);
+      if constexpr (NE == 1) {
+        float xj[4];
+        Pack<float>::unpack(ld16(xs + s * sbb + 16 * i), xj);
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) rt[r4] = fmaf(rem, xj[r4], rt[r4]);
+      } else {
+        uint32_t pc[3];
+        bf16_pieces(rem, pc);
+        const u32x4 rb = {pc[0] | pc[1] << 16, pc[2] | pc[0] << 16, pc[1] | pc[0] << 16, 0u};
+        tot = mfma16x16(ld16(xs + s * sbb + 16 * i), rb, tot, __bf16{});
+      }
     }
     if constexpr (__is_same(T, _Float16)) {  // the operands hold the scales
       f32x4 a[2] = {};
@@ -375,6 +392,14 @@ __global__ __launch_bounds__(WC* KG * 64) __attribute__((amdgpu_waves_per_eu(2, 
     slot = slot == kKvStages - 1 ? 0 : slot + 1;
   }
   wait_vm<0>();
+  if constexpr (NE == 1) {  // row g: its remainders' part from all lane groups
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+      float v = rt[r4] + __shfl_xor(rt[r4], 16);
+      v += __shfl_xor(v, 32);
+      if (g == r4) tot[0] += v;
+    }
+  }
 
   // lane l, value e: row l / 16 + 4 e, column l % 16.  Sums that came out infinite or NaN, again
   // on the fp32 matrix cores (v_mfma_f32_16x16x4: value i of the four lane groups at a time).
