@@ -139,11 +139,19 @@ def _check(status: int, what: str) -> None:
         raise NvfError(f"{what} failed ({status}): {msg}")
 
 
-def _stream() -> int:
-    # torch.cuda.current_stream().cuda_stream without the Stream object: 0.2 us against 2.7,
-    # of the 9 to 12 us that a small call spends on the host (a tensor on the GPU, and so an
-    # initialized torch.cuda, is there by now: the pointers are taken first)
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+def _make_stream(c):
+    """The current stream's handle, as a function.  (A tensor on the GPU, and so an initialized
+    torch.cuda, is there when it is called: the pointers are taken first.)"""
+    # torch.cuda.current_stream().cuda_stream without the Stream object: 0.2 us against 2.7, of the
+    # 9 to 12 us that a small call spends on the host.  Private names: a torch without them takes
+    # the public way.
+    raw_stream, raw_device = getattr(c, "_cuda_getCurrentRawStream", None), getattr(c, "_cuda_getDevice", None)
+    if raw_stream is None or raw_device is None:
+        return lambda: torch.cuda.current_stream().cuda_stream
+    return lambda: raw_stream(raw_device())
+
+
+_stream = _make_stream(torch._C)
 
 
 def _dev(t: torch.Tensor, name: str) -> int:

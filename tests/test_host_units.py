@@ -15,3 +15,15 @@ def test_fastdiv_matches_integer_division():
     r = subprocess.run([str(BIN)], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "0 wrong" in r.stdout
+
+
+def test_stream_without_torchs_private_names(monkeypatch):
+    """A torch that lacks the raw-stream functions: the current stream through the public ones."""
+    import types
+
+    import torch
+
+    from nano_vllm_cpp_amd import ops
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=77))
+    assert ops._make_stream(types.SimpleNamespace())() == 77
